@@ -30,7 +30,7 @@ HIP_FLAGS = [
 ]
 
 ROCM_SOURCES = ["rocm/capi.cpp", "rocm/reduce.hip", "rocm/topk.hip", "rocm/copy.hip",
-                "rocm/softmax.hip", "rocm/loss.hip", "rocm/reduce_bwd.hip"]
+                "rocm/softmax.hip", "rocm/loss.hip", "rocm/reduce_bwd.hip", "rocm/sample.hip"]
 LIB_TPR = os.path.join(PKG, "libtpr_rocm.so")
 LIB_TPR_DEV = os.path.join(PKG, "libtpr_rocm_dev.so")
 
@@ -61,7 +61,8 @@ def _tpr_compiles(force, dev):
     bdir = os.path.join(BUILD, "dev") if dev else BUILD
     os.makedirs(bdir, exist_ok=True)
     inc = ["-I", os.path.join(ROOT, "include"), "-I", os.path.join(CSRC, "rocm")]
-    headers = [os.path.join(ROOT, "include", "tpr_rocm.h"), os.path.join(CSRC, "rocm", "common.h")]
+    headers = [os.path.join(ROOT, "include", "tpr_rocm.h"), os.path.join(CSRC, "rocm", "common.h"),
+               os.path.join(CSRC, "rocm", "select.h")]
     extra = ["-DTPR_DEBUG_KNOBS"] if dev else []
     objs, cmds = [], []
     for src in ROCM_SOURCES:

@@ -58,6 +58,8 @@
 #include <string>
 
 #include "common.h"
+#include "sample.h"
+#include "select.h"
 
 #ifdef TPR_DEBUG_KNOBS
 // Test build only: merge outputs whose row index had to be clamped into the
@@ -93,29 +95,6 @@ constexpr int kWaveCompact = 192;             // per-wave list size that always 
 constexpr int kSlice = 64 * 16;               // elements per wave slice (4 float4 per lane)
 constexpr int kWaveMinSeg = kW * kSlice;      // every wave has a full first slice (8192)
 constexpr long long kWaveMaxSeg = 1LL << 28;  // longest wave-kernel segment (32-bit byte offsets)
-
-// Order-preserving float -> uint32 map: non-negative u -> u | 2^31, negative
-// u -> ~u + 1 (two's-complement negate of the magnitude's image), so -0.0 and
-// +0.0 land on the same key 2^31; every NaN is first made 0x7fc00000 (above
-// +inf).  lmask = 0 keeps the order (largest), ~0 reverses it (smallest).
-// Valid keys are never 0: 0 marks "no element".  Branch-free: one NaN compare
-// (f != f) and select, an arithmetic shift, xor, subtract, xor.
-__device__ __forceinline__ uint32_t f2key_sel(float f, uint32_t lmask) {
-    const uint32_t u = (f != f) ? 0x7fc00000u : __float_as_uint(f);
-    const uint32_t m = (uint32_t)((int32_t)u >> 31);
-    return ((u ^ (m | 0x80000000u)) - m) ^ lmask;
-}
-
-__device__ __forceinline__ uint32_t f2key(float f, int largest) {
-    return f2key_sel(f, largest ? 0u : 0xffffffffu);
-}
-
-// Inverse of f2key.  Exact except for the two canonicalised cases (-0.0 comes
-// back as +0.0, any NaN as 0x7fc00000); callers re-read the input for those.
-__device__ __forceinline__ uint32_t key2bits(uint32_t key, int largest) {
-    const uint32_t k = largest ? key : ~key;
-    return (k & 0x80000000u) ? (k & 0x7fffffffu) : (0u - k);
-}
 
 // Output value of a selected element: from its key, or from the input row when
 // the key cannot tell (+-0.0, NaN payloads).
@@ -186,32 +165,8 @@ __device__ __forceinline__ unsigned long long key64_of(unsigned long long bits, 
     return SortKey<unsigned long long>::of(bits, largest);
 }
 
-__device__ __forceinline__ unsigned long long comp_key(uint32_t key, uint32_t idx) {
-    return ((unsigned long long)key << 32) | (unsigned long long)(0xffffffffu - idx);
-}
-
-__device__ __forceinline__ uint32_t comp_index(unsigned long long c) {
-    return 0xffffffffu - (uint32_t)(c & 0xffffffffull);
-}
-
 // DPP wave reduction from the device library (no LDS round trips).
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) { return __ockl_wfred_max_u32(v); }
-
-// Inclusive prefix sum over the wave's 64 lanes (every lane active): DPP row
-// shifts by 1, 2, 4, 8 (lanes whose source is outside the row add the 0 passed
-// as `old`), then row_bcast:15 and row_bcast:31 carry the row totals upward.
-// No LDS round trips.
-__device__ __forceinline__ int wave_incl_scan(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
-    return v;
-}
-
-__device__ __forceinline__ unsigned long long lanemask_lt() { return (1ull << __lane_id()) - 1ull; }
 
 struct TopkArgs {
     const float* in;
@@ -317,119 +272,15 @@ __device__ void sample_from_sel(const TopkArgs& a, long long row, const float* p
     if (lane == 0) a.ids[row] = (long long)comp_index(sel[pj]);
 }
 
-// Sampling with k > kKMax: the draw of sample_from_sel over a row's sorted top
-// k that tpr_topk has already written (vals[row][k] in rank order, idx[row][k]
-// their indices), one workgroup of NT threads per row.  Thread t owns the
-// contiguous positions [t*per, (t+1)*per): serial sums inside its block, a
-// workgroup scan of the block totals, workgroup minima for the nucleus end m
-// and the drawn position.  p_j is formed with explicit roundings (no
-// contraction), so the three passes over a block see bit-identical c_j.
-constexpr int kDrawNT = 1024;
-
-__device__ __forceinline__ float draw_weight(float v, float temperature, float z0) {
-    return expf(__fsub_rn(__fdiv_rn(v, temperature), z0));
-}
-
-template <int W>
-__device__ __forceinline__ int block_min_i32(int v, int* sh) {
-    v = __ockl_wfred_min_i32(v);
-    if (__lane_id() == 0) sh[threadIdx.x >> 6] = v;
-    __syncthreads();
-    int r = sh[0];
-#pragma unroll
-    for (int q = 1; q < W; ++q) r = min(r, sh[q]);
-    return r;
-}
-
-template <int NT>
-__global__ __launch_bounds__(NT) void k_sample_sorted(const float* vals, const long long* idx, int k,
-                                                      float temperature, float top_p, const float* u,
-                                                      long long* ids) {
-    constexpr int W = NT / 64;
-    __shared__ float wsum[W];
-    __shared__ int wmin[2][W];
-    __shared__ float cm_sh;
-    const long long row = blockIdx.x;
-    const float* v = vals + row * k;
-    const int tid = threadIdx.x, w = tid >> 6;
-    if (!(temperature > 0.0f)) {
-        if (tid == 0) ids[row] = idx[row * k];
-        return;
-    }
-    const int per = (k + NT - 1) / NT;
-    const int j0 = min(k, tid * per), j1 = min(k, j0 + per);
-    const float z0 = __fdiv_rn(v[0], temperature);
-    float s = 0.0f;
-    for (int j = j0; j < j1; ++j) s += draw_weight(v[j], temperature, z0);
-    float incl = s;
-#define TPR_DPP_ADD(CTRL, ROWS) \
-    incl += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(incl), CTRL, ROWS, 0xf, false))
-    TPR_DPP_ADD(0x111, 0xf);  // row_shr:1
-    TPR_DPP_ADD(0x112, 0xf);  // row_shr:2
-    TPR_DPP_ADD(0x114, 0xf);  // row_shr:4
-    TPR_DPP_ADD(0x118, 0xf);  // row_shr:8
-    TPR_DPP_ADD(0x142, 0xa);  // row_bcast:15
-    TPR_DPP_ADD(0x143, 0xc);  // row_bcast:31
-#undef TPR_DPP_ADD
-    if (__lane_id() == 63) wsum[w] = incl;
-    __syncthreads();
-    float before = 0.0f, total = 0.0f;
-#pragma unroll
-    for (int q = 0; q < W; ++q) {
-        const float t = wsum[q];
-        if (q < w) before += t;
-        total += t;
-    }
-    const float excl = before + (incl - s);
-    const float cut = top_p * total;
-    int mj = 0x7fffffff;
-    float c = excl;
-    for (int j = j0; j < j1; ++j) {
-        c += draw_weight(v[j], temperature, z0);
-        if (c >= cut) {
-            mj = j;
-            break;
-        }
-    }
-    mj = block_min_i32<W>(mj, wmin[0]);
-    const int m = (mj == 0x7fffffff) ? k - 1 : mj;
-    if (m >= j0 && m < j1) {
-        c = excl;
-        for (int j = j0; j <= m; ++j) c += draw_weight(v[j], temperature, z0);
-        cm_sh = c;
-    }
-    __syncthreads();
-    const float thr = u[row] * cm_sh;
-    int pj = 0x7fffffff;
-    c = excl;
-    for (int j = j0; j < j1 && j <= m; ++j) {
-        c += draw_weight(v[j], temperature, z0);
-        if (c > thr) {
-            pj = j;
-            break;
-        }
-    }
-    pj = block_min_i32<W>(pj, wmin[1]);
-    if (pj > m) pj = m;
-    if (tid == 0) ids[row] = idx[row * k + pj];
-}
-
-// Workspace of tpr_sample with k > kKMax: tpr_topk's own workspace, then the
-// sorted values [rows][k] (float32) and indices [rows][k] (int64), each part
-// starting on a 256-byte boundary.
-struct SampleSortedLayout {
-    size_t topk_ws, vals_off, idx_off, total;
-};
-
+// Workspace that tpr_sample asks for with k > kKMax: tpr_topk's own, then room
+// for sorted values [rows][k] (float32) and indices [rows][k] (int64), each
+// part on a 256-byte boundary.  The draw no longer sorts, but callers size
+// buffers they keep by this figure and a smaller one stays an error.
 inline size_t round_up_256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-inline SampleSortedLayout sample_sorted_layout(int64_t rows, int64_t cols, int64_t k) {
-    SampleSortedLayout l;
-    l.topk_ws = tpr_topk_workspace_bytes(TPR_FLOAT32, rows, cols, k);
-    l.vals_off = round_up_256(l.topk_ws);
-    l.idx_off = l.vals_off + round_up_256((size_t)rows * (size_t)k * sizeof(float));
-    l.total = l.idx_off + (size_t)rows * (size_t)k * sizeof(long long);
-    return l;
+inline size_t sample_sorted_bytes(int64_t rows, int64_t cols, int64_t k) {
+    return round_up_256(tpr_topk_workspace_bytes(TPR_FLOAT32, rows, cols, k)) +
+           round_up_256((size_t)rows * (size_t)k * sizeof(float)) + (size_t)rows * (size_t)k * sizeof(long long);
 }
 
 // Small shared state of the workgroup-level helpers.
@@ -1410,17 +1261,6 @@ __device__ __forceinline__ uint32_t group_max(uint32_t v) {
     return v;
 }
 
-template <int M, int P>
-__device__ __forceinline__ void sort_lane_stage(unsigned long long (&x)[P], bool keep_max) {
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-        const uint32_t lo = xor_lane<M>((uint32_t)x[p]);
-        const uint32_t hi = xor_lane<M>((uint32_t)(x[p] >> 32));
-        const unsigned long long y = ((unsigned long long)hi << 32) | lo;
-        x[p] = ((x[p] > y) == keep_max) ? x[p] : y;
-    }
-}
-
 // Descending bitonic sort of 64 * P composites held P per lane across one
 // wave (lane l holds positions l*P .. l*P+P-1): lane permutes for distances of
 // at least P, compare-exchanges in registers below.
@@ -2381,67 +2221,6 @@ __device__ int block_prefix_excl(int v, int* wtot, int& total) {
     return before + inc - v;
 }
 
-// Descending bitonic sort of n composites (n / P threads, a multiple of 64,
-// at most NT) held P per thread: thread t holds positions t*P .. t*P+P-1.
-// Distances below P: compare-exchanges in registers; below 64*P: the partner
-// lane's value by a lane permute; the rest through xb (LDS, NT*min(P, 4)
-// composites) with a barrier, which every thread of the workgroup reaches.
-template <int NT, int P>
-__device__ void reg_sort_desc(unsigned long long (&x)[P], unsigned long long* xb, int n) {
-    constexpr int Q = P < 4 ? P : 4;
-    const int t = threadIdx.x;
-    const bool active = t < n / P;  // whole waves
-    for (int s = 2; s <= n; s <<= 1) {
-        for (int d = s >> 1; d >= P; d >>= 1) {
-            const int m = d / P;  // partner thread t ^ m
-            const bool desc = ((t * P) & s) == 0;
-            const bool keep_max = ((t & m) == 0) == desc;
-            if (!active && m < 64) continue;
-            switch (m) {
-                case 1: sort_lane_stage<1, P>(x, keep_max); break;
-                case 2: sort_lane_stage<2, P>(x, keep_max); break;
-                case 4: sort_lane_stage<4, P>(x, keep_max); break;
-                case 8: sort_lane_stage<8, P>(x, keep_max); break;
-                case 16: sort_lane_stage<16, P>(x, keep_max); break;
-                case 32: sort_lane_stage<32, P>(x, keep_max); break;
-                default:
-#pragma unroll
-                    for (int p0 = 0; p0 < P; p0 += Q) {
-                        if (active) {
-#pragma unroll
-                            for (int q = 0; q < Q; ++q) xb[q * NT + t] = x[p0 + q];
-                        }
-                        __syncthreads();
-                        if (active) {
-#pragma unroll
-                            for (int q = 0; q < Q; ++q) {
-                                const unsigned long long y = xb[q * NT + (t ^ m)];
-                                x[p0 + q] = ((x[p0 + q] > y) == keep_max) ? x[p0 + q] : y;
-                            }
-                        }
-                        __syncthreads();
-                    }
-            }
-        }
-        if (!active) continue;
-#pragma unroll
-        for (int dd = P / 2; dd >= 1; dd >>= 1) {
-            if (dd < s) {
-#pragma unroll
-                for (int p = 0; p < P; ++p) {
-                    if ((p & dd) == 0) {
-                        const bool desc = ((t * P + p) & s) == 0;
-                        const unsigned long long u = x[p], v = x[p + dd];
-                        const bool sw = (u > v) != desc;
-                        x[p] = sw ? v : u;
-                        x[p + dd] = sw ? u : v;
-                    }
-                }
-            }
-        }
-    }
-}
-
 template <int NT, int P>
 struct RselShared {
     static constexpr int kBuf = (NT * (P < 4 ? P : 4) > 1024) ? NT * (P < 4 ? P : 4) : 1024;
@@ -3364,7 +3143,7 @@ int tpr_topk(const void* in, int32_t dtype, int64_t rows, int64_t cols, int64_t 
 
 size_t tpr_sample_workspace_bytes(int32_t dtype, int64_t rows, int64_t cols, int64_t k) {
     if (dtype == TPR_FLOAT32 && k > tpr::kKMax && k <= cols && rows > 0 && cols <= 0x7fffffffLL)
-        return tpr::sample_sorted_layout(rows, cols, k).total;
+        return tpr::sample_sorted_bytes(rows, cols, k);
     return tpr_topk_workspace_bytes(dtype, rows, cols, k);
 }
 
@@ -3384,23 +3163,15 @@ int tpr_sample(const void* logits, int32_t dtype, int64_t rows, int64_t cols, in
     smp.u = uniforms;
     smp.ids = reinterpret_cast<long long*>(out_ids);
     if (k > kKMax) {
-        // the sorted top k through tpr_topk into the workspace, then the draw
-        // by one workgroup per row
+        // no sort: the nucleus end and the draw by weight (sample.hip).  The
+        // workspace is still asked for, but not written.
         if (cols > 0x7fffffffLL) return fail(TPR_ERR_NOT_IMPLEMENTED, "tpr_sample: rows longer than 2^31-1");
         if (rows > 0x7fffffffLL) return fail(TPR_ERR_NOT_IMPLEMENTED, "tpr_sample: more than 2^31-1 rows");
-        const SampleSortedLayout l = sample_sorted_layout(rows, cols, k);
-        if (workspace == nullptr || workspace_bytes < l.total)
-            return fail(TPR_ERR_WORKSPACE, "tpr_sample: workspace too small (need " + std::to_string(l.total) +
-                                               " bytes)");
-        char* ws = static_cast<char*>(workspace);
-        float* vals = reinterpret_cast<float*>(ws + l.vals_off);
-        long long* idx = reinterpret_cast<long long*>(ws + l.idx_off);
-        const int rc = topk_launch(logits, dtype, rows, cols, row_stride, k, 1, vals, idx,
-                                   l.topk_ws ? workspace : nullptr, l.topk_ws, stream, nullptr);
-        if (rc != TPR_OK) return rc;
-        hipLaunchKernelGGL((k_sample_sorted<kDrawNT>), dim3((unsigned)rows), dim3(kDrawNT), 0,
-                           static_cast<hipStream_t>(stream), vals, idx, (int)k, temperature, top_p, uniforms, smp.ids);
-        return check_launch("tpr_sample");
+        const size_t need = sample_sorted_bytes(rows, cols, k);
+        if (workspace == nullptr || workspace_bytes < need)
+            return fail(TPR_ERR_WORKSPACE, "tpr_sample: workspace too small (need " + std::to_string(need) + " bytes)");
+        return sample_rows(static_cast<const float*>(logits), rows, cols, row_stride, k, temperature, top_p, uniforms,
+                           smp.ids, static_cast<hipStream_t>(stream));
     }
     return topk_launch(logits, dtype, rows, cols, row_stride, k, 1, nullptr, nullptr, workspace, workspace_bytes,
                        stream, &smp);
