@@ -98,4 +98,18 @@ __device__ __forceinline__ float xor_lane_f(float v, int m) {
     }
 }
 
+// The same exchange for any type of whole 32-bit words (every lane active, m a
+// power of two up to 32 that is known when the caller's loop unrolls).
+template <class T>
+__device__ __forceinline__ T lane_xor(T v, int m) {
+    static_assert(sizeof(T) % 4 == 0, "whole 32-bit words");
+    uint32_t w[sizeof(T) / 4];
+    __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) / 4); ++i) w[i] = __float_as_uint(xor_lane_f(__uint_as_float(w[i]), m));
+    T r;
+    __builtin_memcpy(&r, w, sizeof(T));
+    return r;
+}
+
 }  // namespace tpr

@@ -16,6 +16,8 @@
 // adjacent dims that are contiguous with each other and share reduce status):
 //   rows    [K, R]     R contiguous          -> k_rows   (128-bit loads along rows)
 //   cols    [K1, R, K2] K2 contiguous         -> k_cols   (128-bit loads along K2)
+//   runs    several reduced dims, or kept dims that do not merge, the innermost
+//           reduced dim contiguous            -> k_runs   (128-bit loads along the runs)
 //   general anything else                    -> k_general (index arithmetic)
 // Any of them may split the reduced extent over S workgroups; the S partial
 // states then go through k_finalize (no atomics; fixed combine order, so results
@@ -60,7 +62,7 @@ struct SumOp {
     __device__ static State state(Acc a) { return {a}; }
     __device__ static State identity() { return {0.0}; }
     __device__ static State comb(State a, State b) { return {a.s + b.s}; }
-    __device__ static State shfl(State s, int m) { return {__shfl_xor(s.s, m, kWave)}; }
+    __device__ static State shfl(State s, int m) { return {lane_xor(s.s, m)}; }
 };
 
 // Product in fp64 (the reference multiplies in the output dtype, :424-427).
@@ -75,7 +77,7 @@ struct ProdOp {
     __device__ static State state(Acc a) { return {a}; }
     __device__ static State identity() { return {1.0}; }
     __device__ static State comb(State a, State b) { return {a.s * b.s}; }
-    __device__ static State shfl(State s, int m) { return {__shfl_xor(s.s, m, kWave)}; }
+    __device__ static State shfl(State s, int m) { return {lane_xor(s.s, m)}; }
 };
 
 // Sum of |x|^p in fp64 (norm_kernel's abs().pow(p).sum(), :858-872).  KIND 1:
@@ -96,7 +98,7 @@ struct NormOp {
     __device__ static State state(Acc a) { return {a}; }
     __device__ static State identity() { return {0.0}; }
     __device__ static State comb(State a, State b) { return {a.s + b.s}; }
-    __device__ static State shfl(State s, int m) { return {__shfl_xor(s.s, m, kWave)}; }
+    __device__ static State shfl(State s, int m) { return {lane_xor(s.s, m)}; }
 };
 
 // all / any: an element is true when x != 0 (NaN is true, -0.0 is false), as
@@ -117,7 +119,7 @@ struct BoolOp {
     __device__ static State state(Acc a) { return {a}; }
     __device__ static State identity() { return {ANY ? 0 : 1}; }
     __device__ static State comb(State a, State b) { return {ANY ? (a.b | b.b) : (a.b & b.b)}; }
-    __device__ static State shfl(State s, int m) { return {__shfl_xor(s.b, m, kWave)}; }
+    __device__ static State shfl(State s, int m) { return {lane_xor(s.b, m)}; }
 };
 
 struct ArgS { float v; long long i; };
@@ -155,7 +157,7 @@ struct ArgOp {
         return t ? b : a;
     }
     __device__ static State shfl(State s, int m) {
-        return {__shfl_xor(s.v, m, kWave), __shfl_xor(s.i, m, kWave)};
+        return {lane_xor(s.v, m), lane_xor(s.i, m)};
     }
 };
 
@@ -196,8 +198,56 @@ struct WelfordOp {
         return {n, a.mean + d * f, a.m2 + b.m2 + d * d * a.n * f};
     }
     __device__ static State shfl(State s, int m) {
-        return {__shfl_xor(s.n, m, kWave), __shfl_xor(s.mean, m, kWave),
-                __shfl_xor(s.m2, m, kWave)};
+        return {lane_xor(s.n, m), lane_xor(s.mean, m),
+                lane_xor(s.m2, m)};
+    }
+};
+
+// var / std as sums shifted by one element K of the reduced set (acc's last
+// argument), the same for every thread of an output: the states of all threads
+// and splits add up, without WelfordOp's select per element and its merges
+// with a divide each.  K's own term is in M2, so n (K - mean)^2 <= n M2 and the
+// cancellation in S2 - S1^2 / n costs at most about n 2^-53 of M2: the planner
+// takes it for sets of at most kShiftMax elements (2e-9 there), below float32's
+// rounding.
+constexpr long long kShiftMax = 1LL << 24;
+struct ShiftS { double s1, s2; int n, pad; };
+
+struct ShiftVarOp {
+    static constexpr bool kIndexed = false;
+    using Acc = ShiftS;
+    using State = ShiftS;
+    using Wide = WelfordOp;
+    __device__ static Acc init() { return {0.0, 0.0, 0, 0}; }
+    template <class I>
+    __device__ static void acc(Acc& a, float x, I, float k) {
+        const double d = (double)x - (double)k;
+        a.s1 += d;
+        a.s2 = fma(d, d, a.s2);
+        a.n += 1;
+    }
+    __device__ static State state(Acc a) { return a; }
+    __device__ static State identity() { return {0.0, 0.0, 0, 0}; }
+    __device__ static State comb(State a, State b) { return {a.s1 + b.s1, a.s2 + b.s2, a.n + b.n, 0}; }
+    __device__ static State shfl(State s, int m) { return {lane_xor(s.s1, m), lane_xor(s.s2, m), lane_xor(s.n, m), 0}; }
+};
+
+// What a workgroup's state becomes before it is written or merged with other
+// splits': the state itself, or ShiftVarOp's sums as a WelfordOp state.
+template <class Op>
+struct Finish {
+    using Final = Op;
+    static constexpr bool kShift = false;
+    __device__ static typename Op::State of(typename Op::State s, float) { return s; }
+};
+template <>
+struct Finish<ShiftVarOp> {
+    using Final = WelfordOp;
+    static constexpr bool kShift = true;
+    __device__ static WelS of(ShiftS s, float k) {
+        if (s.n == 0) return {0.0, 0.0, 0.0};
+        const double n = (double)s.n, m = s.s1 / n;
+        return {n, (double)k + m, fmax(0.0, s.s2 - s.s1 * m)};
     }
 };
 
@@ -830,6 +880,139 @@ __global__ __launch_bounds__(kBlock) void k_general(GenArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// Run kernel: reduced elements that lie in Q contiguous runs of L elements at
+// run offsets given by the outer reduced dims (channel statistics of
+// [N, C, H, W]: N runs of H*W per channel), any kept dims.  A run is cut into
+// nch chunks; units (run, chunk) go round robin to groups of G = 2^gsh lanes,
+// NV-element vectors along the chunk (starting at any element), eight vectors
+// in flight per lane: from one chunk, or one each from eight runs where a run
+// is a single vector per lane.  blockIdx.x = output * S + split; the S
+// splits of an output finish in the same launch (split_finish) or through
+// k_finalize.  Index arithmetic is per run, not per element as in k_general.
+// MI355X, [64, 64, 56, 56] over dims 0, 2, 3 (51 MB, 7.4 us at the read rate):
+// sum 43 -> 14.3 us against k_general, var 52 -> 15.7; [16, 1024, 2048] over 0,
+// 2 (134 MB, 19.5 us) sum 26.8.  What bounds it: two memory latencies, the
+// workgroup combine and, where an output is split, the exchange.
+// ---------------------------------------------------------------------------
+struct RunArgs {
+    const void* in;
+    int nk, nr;  // kept dims; outer reduced dims
+    long long ksz[TPR_MAX_DIMS], kst[TPR_MAX_DIMS], rst[TPR_MAX_DIMS];
+    unsigned rsz[TPR_MAX_DIMS];
+    int L, chunk;
+    unsigned units, nch;
+    int gsh, S;
+    long long nout;
+    void* out;
+    void* part;
+    Fin fin;
+    unsigned* tickets;
+};
+
+// NV elements of type T starting at any element.
+template <class T, int NV>
+struct AnyVec {
+    typedef T type __attribute__((ext_vector_type(NV), aligned(sizeof(T))));
+};
+
+template <class Op, class T, int NV, int BLK>
+__global__ __launch_bounds__(BLK) void k_runs(RunArgs a) {
+    using Acc = typename Op::Acc;
+    using Final = typename Finish<Op>::Final;
+    using State = typename Final::State;
+    using V = typename AnyVec<T, NV>::type;
+    constexpr int U = 8;  // vectors in flight per lane
+    const long long o = blockIdx.x / a.S;
+    const int s = blockIdx.x % a.S;
+    long long base = 0;
+    {
+        long long rem = o;
+        for (int d = a.nk - 1; d > 0; --d) {
+            base += (rem % a.ksz[d]) * a.kst[d];
+            rem /= a.ksz[d];
+        }
+        if (a.nk > 0) base += rem * a.kst[0];
+    }
+    const T* in = static_cast<const T*>(a.in) + base;
+    float prm = a.fin.p;
+    if constexpr (Finish<Op>::kShift) prm = in[0];  // one shift for all splits of the output
+    auto run_at = [&](unsigned q) {
+        long long off = 0;
+        for (int d = a.nr - 1; d > 0; --d) {
+            off += (long long)(q % a.rsz[d]) * a.rst[d];
+            q /= a.rsz[d];
+        }
+        return in + (a.nr > 0 ? off + (long long)q * a.rst[0] : off);
+    };
+    const int G = 1 << a.gsh;  // >= NV: an unfinished vector is one element per lane
+    const int l = threadIdx.x & (G - 1);
+    const unsigned ngrp = (unsigned)(a.S * BLK) >> a.gsh;
+    const unsigned gid = (unsigned)(s * BLK + (int)threadIdx.x) >> a.gsh;
+    Acc acc = Op::init();
+    if (a.nch == 1 && a.L / NV <= G) {
+        const int nv = a.L / NV;
+        const int lv = min(l, nv - 1);
+        const int te = min(nv * NV + l, a.L - 1);
+        for (unsigned u = gid; u < a.units; u += U * ngrp) {
+            V x[U];
+            T t[U];
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
+                const T* p = run_at(min(u + k * ngrp, a.units - 1));
+                if (nv > 0) x[k] = *reinterpret_cast<const V*>(p + lv * NV);
+                t[k] = p[te];
+            }
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
+                const unsigned q = u + k * ngrp;
+                if (q < a.units) {
+                    const int j = (int)q * a.L;
+                    if (l < nv) {
+#pragma unroll
+                        for (int i = 0; i < NV; ++i) Op::acc(acc, (T)x[k][i], j + l * NV + i, prm);
+                    }
+                    if (nv * NV + l < a.L) Op::acc(acc, t[k], j + te, prm);
+                }
+            }
+        }
+    } else {
+        for (unsigned u = gid; u < a.units; u += ngrp) {
+            const unsigned q = u / a.nch;
+            const int e0 = (int)(u - q * a.nch) * a.chunk;
+            const int len = min(a.chunk, a.L - e0);
+            const T* p = run_at(q) + e0;
+            const int j = (int)q * a.L + e0;
+            const int nv = len / NV;
+            const int te = min(nv * NV + l, len - 1);
+            const T t = p[te];
+            for (int v = l; v < nv; v += U * G) {
+                V x[U];
+#pragma unroll
+                for (int k = 0; k < U; ++k) x[k] = *reinterpret_cast<const V*>(p + (long long)min(v + k * G, nv - 1) * NV);
+#pragma unroll
+                for (int k = 0; k < U; ++k) {
+                    if (v + k * G < nv) {
+#pragma unroll
+                        for (int i = 0; i < NV; ++i) Op::acc(acc, (T)x[k][i], j + (v + k * G) * NV + i, prm);
+                    }
+                }
+            }
+            if (nv * NV + l < len) Op::acc(acc, t, j + te, prm);
+        }
+    }
+    const State st = Finish<Op>::of(block_reduce_n<Op, BLK>(Op::state(acc)), prm);
+    if (a.tickets) {
+        split_finish<Final, BLK>(st, reinterpret_cast<State*>(a.part), a.tickets + o, a.S, s, a.nout, o,
+                              [&](const State& r) { fin_write(r, a.fin, a.out, o); });
+        return;
+    }
+    if (threadIdx.x == 0) {
+        if (a.S == 1) fin_write(st, a.fin, a.out, o);
+        else reinterpret_cast<State*>(a.part)[(long long)s * a.nout + o] = st;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Finalize: combine S partial states per output in split order.
 // ---------------------------------------------------------------------------
 struct FinArgs {
@@ -865,7 +1048,7 @@ __global__ __launch_bounds__(kBlock) void k_finalize_block(FinArgs a) {
 // ---------------------------------------------------------------------------
 // Host planner.
 // ---------------------------------------------------------------------------
-enum PlanKind { P_ROWS = 1, P_COLS = 2, P_GENERAL = 3 };
+enum PlanKind { P_ROWS = 1, P_COLS = 2, P_GENERAL = 3, P_RUNS = 4 };
 
 struct Plan {
     int kind = P_GENERAL;
@@ -892,6 +1075,8 @@ struct Plan {
     int nk = 0, nr = 0;
     long long ksz[TPR_MAX_DIMS], kst[TPR_MAX_DIMS], rsz[TPR_MAX_DIMS], rst[TPR_MAX_DIMS];
     long long nout = 1, count = 1;
+    int gsh = 6;                              // runs: log2 of the lanes per run
+    long long L = 1, units = 1, nch = 1, rchunk = 1;  // runs
 };
 
 bool norm_is_inf(double p) { return std::isinf(p); }
@@ -1022,6 +1207,32 @@ int validate(const tpr_reduce_desc* d) {
     return TPR_OK;
 }
 
+// Splits, lanes per run and chunks of a run plan for NV-element vectors.  512
+// threads per workgroup with eight vectors in flight per lane; an output is
+// split only when the outputs alone leave CUs without a workgroup, into about
+// 1.5 workgroups per CU: more, smaller ones lose to the split's counters, whose
+// atomics on neighbouring words take about 9 ns each (MI355X, us, sums over 0,
+// 2, 3: [64, 64, 56, 56] S = 2 20, 4 15.0, 8 14.3, 32 25; [128, 256, 14, 14]
+// S = 1 7.6, 2 8.9, 8 14).  One wave per output where an output has few
+// elements.  As many units (run, chunk) as there are lane groups, so that none
+// of them idles.
+void plan_runs(Plan& p, int NV) {
+    const long long cus = device_info().cus;
+    const long long Q = p.count / p.L;
+    const long long vecs = ceil_div(p.L, NV);
+    p.colblock = p.count <= 2048 ? kWave : 512;
+    p.gsh = NV >= 16 ? 4 : NV == 8 ? 3 : 2;
+    while (p.gsh < 6 && (1LL << p.gsh) < vecs) ++p.gsh;
+    const long long G = 1LL << p.gsh;
+    p.S = p.nout < cus ? std::min(ceil_div(cus * 3 / 2, p.nout), std::max(1LL, p.count / 4096)) : 1;
+    if (knobs().splits > 0) p.S = std::min((long long)knobs().splits, p.count);
+    const long long groups = p.S * p.colblock / G;
+    p.nch = std::min(ceil_div(p.L, NV * G), std::max(ceil_div(groups, Q), ceil_div(p.L, 16384)));
+    p.rchunk = ceil_div(ceil_div(p.L, p.nch), NV) * NV;
+    p.nch = ceil_div(p.L, p.rchunk);
+    p.units = Q * p.nch;
+}
+
 Plan make_plan(const tpr_reduce_desc* d, const void* in) {
     Plan p;
     p.state_bytes = state_size(d->op, d->p);
@@ -1063,6 +1274,32 @@ Plan make_plan(const tpr_reduce_desc* d, const void* in) {
     }
     Dims K, Rd;
     for (auto& x : dims) (x.red ? Rd : K).push_back(x);
+    // Where the result does not depend on the order of the reduced elements
+    // (not argmax/argmin, nor the sign of a zero extremum of a float amax/amin)
+    // the reduced dims are visited in memory order, whatever the view's.
+    const bool ordered = d->op == TPR_ARGMAX || d->op == TPR_ARGMIN ||
+                         ((d->op == TPR_AMAX || d->op == TPR_AMIN || d->op == TPR_NORM) &&
+                          (d->in_dtype == TPR_FLOAT32 || d->in_dtype == TPR_FLOAT64));
+    if (!ordered)
+        std::stable_sort(Rd.d, Rd.d + Rd.n,
+                         [](const Dim& x, const Dim& y) { return std::llabs(x.stride) > std::llabs(y.stride); });
+    // Kept (and reduced) dims that continue each other merge across whatever
+    // lay between them: outputs are row-major over the kept dims, and reduced
+    // indices over the reduced dims.
+    auto merge = [](Dims& v) {
+        Dims m;
+        for (auto& x : v) {
+            if (!m.empty() && m.back().stride == x.stride * x.size) {
+                m.back().size *= x.size;
+                m.back().stride = x.stride;
+            } else {
+                m.push_back(x);
+            }
+        }
+        v = m;
+    };
+    merge(K);
+    merge(Rd);
 
     const auto& dev = device_info();
     const bool aligned16 = (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
@@ -1098,7 +1335,7 @@ Plan make_plan(const tpr_reduce_desc* d, const void* in) {
         Rfull = Rd[0].size;
         Rd[0].size = kChunk;  // plan one chunk; the general kernel takes the whole run back
     }
-    const bool int_ok = Rd.empty() || (Rd.size() == 1 && Rd[0].size < kIntMax);
+    const bool int_ok = Rd.empty() || (Rd.size() == 1 ? Rd[0].size : p.count) < kIntMax;
     if (empty || force_general || !int_ok) {
         fill_general();
     } else if (K.size() <= 1 && (Rd.empty() || (Rd.size() == 1 && Rd[0].stride == 1))) {
@@ -1164,10 +1401,8 @@ Plan make_plan(const tpr_reduce_desc* d, const void* in) {
                 p.S = 1;
             }
         }
-    } else if (!K.empty() && K.back().stride == 1 && Rd.size() == 1 &&
-               (K.size() == 1 ? true : (K.size() == 2)) &&
-               (K.size() == 1 ? (dims.front().red) : (dims.size() == 3 && dims[1].red))) {
-        // cols: [K1?, R, K2] with K2 contiguous
+    } else if (!K.empty() && K.back().stride == 1 && Rd.size() == 1 && K.size() <= 2) {
+        // cols: [K1?, R, K2] with K2 contiguous (R may lie anywhere in the view)
         p.kind = P_COLS;
         p.inner = K.back().size;
         p.outer = (K.size() == 2) ? K[0].size : 1;
@@ -1197,6 +1432,15 @@ Plan make_plan(const tpr_reduce_desc* d, const void* in) {
         if (threads < target) S = std::min(ceil_div(target, threads), std::max(1LL, p.R / (ty * 8)));
         if (knobs().splits > 0) S = knobs().splits;
         p.S = std::max(1LL, std::min(S, ceil_div(p.R, ty)));
+    } else if (!Rd.empty() && Rd.back().stride == 1 && Rd.back().size >= 4 && p.count < kIntMax) {
+        // runs: the innermost reduced dim contiguous
+        p.kind = P_RUNS;
+        p.nk = (int)K.size();
+        p.nr = (int)Rd.size() - 1;
+        for (int i = 0; i < p.nk; ++i) { p.ksz[i] = K[i].size; p.kst[i] = K[i].stride; }
+        for (int i = 0; i < p.nr; ++i) { p.rsz[i] = Rd[i].size; p.rst[i] = Rd[i].stride; }
+        p.L = Rd.back().size;
+        plan_runs(p, 4);
     } else {
         fill_general();
     }
@@ -1336,6 +1580,34 @@ int launch_general(const Plan& p, const float* in, void* out, void* ws, Fin fin,
     return check_launch("k_general");
 }
 
+template <class Op, class T, int NV>
+int launch_runs(const Plan& p, const void* in, void* out, void* ws, Fin fin, hipStream_t st, unsigned* tickets) {
+    RunArgs a;
+    a.in = in;
+    a.nk = p.nk;
+    a.nr = p.nr;
+    for (int i = 0; i < TPR_MAX_DIMS; ++i) {
+        a.ksz[i] = i < p.nk ? p.ksz[i] : 1;
+        a.kst[i] = i < p.nk ? p.kst[i] : 0;
+        a.rsz[i] = i < p.nr ? (unsigned)p.rsz[i] : 1u;
+        a.rst[i] = i < p.nr ? p.rst[i] : 0;
+    }
+    a.L = (int)p.L;
+    a.chunk = (int)p.rchunk;
+    a.units = (unsigned)p.units;
+    a.nch = (unsigned)p.nch;
+    a.gsh = p.gsh;
+    a.S = (int)p.S;
+    a.nout = p.nout;
+    a.out = out;
+    a.part = ws;
+    a.fin = fin;
+    a.tickets = tickets;
+    if (p.colblock == kWave) hipLaunchKernelGGL((k_runs<Op, T, NV, kWave>), dim3(p.nout * p.S), dim3(kWave), 0, st, a);
+    else hipLaunchKernelGGL((k_runs<Op, T, NV, 512>), dim3(p.nout * p.S), dim3(512), 0, st, a);
+    return check_launch("k_runs");
+}
+
 template <class Op>
 int launch_finalize(const Plan& p, void* out, const void* ws, Fin fin, hipStream_t st) {
     FinArgs a{ws, p.nout, (int)p.S, out, fin};
@@ -1373,11 +1645,13 @@ int run_chunks(const Plan& p, const void* in, size_t esize, void* out, void* ws,
 unsigned* stream_tickets(hipStream_t st);
 
 // Counters for a split plan that finishes in its own launch (split_finish):
-// row plans with S > 1 and one row per workgroup, on a stream that has a
-// counter block.  Null: the plan takes the separate finalize launch.
+// row plans with S > 1 and one row per workgroup and run plans with S > 1, on a
+// stream that has a counter block.  Null: the plan takes the separate finalize
+// launch.
 unsigned* fused_split_tickets(const Plan& p, hipStream_t st) {
-    if (p.kind != P_ROWS || p.S <= 1 || p.nchunk > 1 || p.partial || p.lanes < kBlock || p.reg_wpr > 0 ||
-        p.var_nv > 0 || p.rows > kTicketsPerStream)
+    if (p.S <= 1 || p.nchunk > 1 || p.partial) return nullptr;
+    if (p.kind == P_RUNS) return p.nout <= kTicketsPerStream ? stream_tickets(st) : nullptr;
+    if (p.kind != P_ROWS || p.lanes < kBlock || p.reg_wpr > 0 || p.var_nv > 0 || p.rows > kTicketsPerStream)
         return nullptr;
     return stream_tickets(st);
 }
@@ -1393,6 +1667,14 @@ int run(const Plan& p, const float* in, void* out, void* ws, Fin fin, hipStream_
     unsigned* tk = fused_split_tickets(p, st);
     if (p.kind == P_ROWS) rc = launch_rows<Op>(p, in, out, ws, fin, st, tk);
     else if (p.kind == P_COLS) rc = launch_cols<Op>(p, in, out, ws, fin, st);
+    else if (p.kind == P_RUNS) {
+        if constexpr (std::is_same<Op, WelfordOp>::value) {
+            rc = p.count <= kShiftMax ? launch_runs<ShiftVarOp, float, 4>(p, in, out, ws, fin, st, tk)
+                                      : launch_runs<Op, float, 4>(p, in, out, ws, fin, st, tk);
+        } else {
+            rc = launch_runs<Op, float, 4>(p, in, out, ws, fin, st, tk);
+        }
+    }
     else rc = launch_general<Op>(p, in, out, ws, fin, st);
     if (rc != TPR_OK) return rc;
     if (p.S > 1 && !tk) rc = launch_finalize<Op>(p, out, ws, fin, st);
@@ -1432,7 +1714,7 @@ struct IntSumOp {
     __device__ static State state(Acc a) { return {a}; }
     __device__ static State identity() { return {PROD ? 1 : 0}; }
     __device__ static State comb(State a, State b) { return {PROD ? wrap_mul(a.s, b.s) : wrap_add(a.s, b.s)}; }
-    __device__ static State shfl(State s, int m) { return {__shfl_xor(s.s, m, kWave)}; }
+    __device__ static State shfl(State s, int m) { return {lane_xor(s.s, m)}; }
 };
 
 // Mean of an integer input: the reference converts the input to Float32 first
@@ -1451,7 +1733,7 @@ struct IntMeanOp {
     __device__ static State state(Acc a) { return {a}; }
     __device__ static State identity() { return {0.0}; }
     __device__ static State comb(State a, State b) { return {a.s + b.s}; }
-    __device__ static State shfl(State s, int m) { return {__shfl_xor(s.s, m, kWave)}; }
+    __device__ static State shfl(State s, int m) { return {lane_xor(s.s, m)}; }
 };
 
 // Order-preserving signed 64-bit key of an integer element: the value itself,
@@ -1501,7 +1783,7 @@ struct IntArgOp {
         t = t || (b.v == a.v && b.i < a.i);
         return t ? b : a;
     }
-    __device__ static State shfl(State s, int m) { return {__shfl_xor(s.v, m, kWave), __shfl_xor(s.i, m, kWave)}; }
+    __device__ static State shfl(State s, int m) { return {lane_xor(s.v, m), lane_xor(s.i, m)}; }
 };
 
 template <class T, bool ANY>
@@ -1519,7 +1801,7 @@ struct IntBoolOp {
     __device__ static State state(Acc a) { return {a}; }
     __device__ static State identity() { return {ANY ? 0 : 1}; }
     __device__ static State comb(State a, State b) { return {ANY ? (a.b | b.b) : (a.b & b.b)}; }
-    __device__ static State shfl(State s, int m) { return {__shfl_xor(s.b, m, kWave)}; }
+    __device__ static State shfl(State s, int m) { return {lane_xor(s.b, m)}; }
 };
 
 __device__ __forceinline__ void fin_write(const SumI& s, const Fin&, void* out, long long o) {
@@ -1809,7 +2091,7 @@ struct F64SumOp {
     __device__ static State state(Acc a) { return {a}; }
     __device__ static State identity() { return {PROD ? 1.0 : 0.0}; }
     __device__ static State comb(State a, State b) { return {PROD ? a.s * b.s : a.s + b.s}; }
-    __device__ static State shfl(State s, int m) { return {__shfl_xor(s.s, m, kWave)}; }
+    __device__ static State shfl(State s, int m) { return {lane_xor(s.s, m)}; }
 };
 
 template <int KIND>  // 1: |x|, 2: x*x, 0: pow(|x|, p)
@@ -1828,7 +2110,7 @@ struct F64NormOp {
     __device__ static State state(Acc a) { return {a}; }
     __device__ static State identity() { return {0.0}; }
     __device__ static State comb(State a, State b) { return {a.s + b.s}; }
-    __device__ static State shfl(State s, int m) { return {__shfl_xor(s.s, m, kWave)}; }
+    __device__ static State shfl(State s, int m) { return {lane_xor(s.s, m)}; }
 };
 
 struct ArgSD { double v; long long i; };
@@ -1855,7 +2137,7 @@ struct F64ArgOp {
         t = t || (b.v == a.v && b.i < a.i);
         return t ? b : a;
     }
-    __device__ static State shfl(State s, int m) { return {__shfl_xor(s.v, m, kWave), __shfl_xor(s.i, m, kWave)}; }
+    __device__ static State shfl(State s, int m) { return {lane_xor(s.v, m), lane_xor(s.i, m)}; }
 };
 
 struct WelAccD { double k; long long n; double s1, s2; };
@@ -1955,6 +2237,8 @@ void adapt_plan_int(Plan& p, const tpr_reduce_desc* d, const void* in, int es) {
         if (threads < target) S = std::min(ceil_div(target, threads), std::max(1LL, p.R / (ty * 8)));
         if (knobs().splits > 0) S = knobs().splits;
         p.S = std::max(1LL, std::min(S, ceil_div(p.R, ty)));
+    } else if (p.kind == P_RUNS) {
+        plan_runs(p, NV);
     }
     p.ws = (p.S > 1 || p.nchunk > 1) ? (size_t)(p.S * p.nchunk) * (size_t)p.nout * p.state_bytes : 0;
 }
@@ -2001,6 +2285,8 @@ int launch_int_layout(const Plan& p, const void* in, void* out, void* ws, Fin fi
         else TPR_COLS_I(64)
         else return fail(TPR_ERR_INVALID_ARG, "tpr_reduce: tx must be 64, 128 or 256");
 #undef TPR_COLS_I
+    } else if (p.kind == P_RUNS) {
+        return launch_runs<Op, T, NV>(p, in, out, ws, fin, st, tickets);
     } else {
         GenArgsI a{};
         a.in = in; a.nk = p.nk; a.nr = p.nr;
