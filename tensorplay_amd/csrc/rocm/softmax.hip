@@ -14,10 +14,12 @@
 //
 // The reference materialises max, shifted, exp and sum tensors (five passes
 // and three temporaries).  Here one kernel does it:
-//   * rows shorter than 16384 floats (or a few long rows, up to 32768)
+//   * rows shorter than 16384 floats (or a few long rows, up to 32768), starting
+//     and ending at any float,
 //     stay in registers: read once and written once -- k_smx_rows;
 //   * forward rows of 16385..655360 floats with more rows than CUs and two
-//     pieces or more per row, and every forward row of 153601..655360, are
+//     pieces or more per row, every forward row of 153601..655360 and every
+//     row of those lengths that does not start and end on 16 bytes, are
 //     cut into pieces held in registers by one workgroup each, (max, sum
 //     exp) exchanged -- k_smx_fwd_pieces;
 //   * rows of 16384..153600 floats, at least one per CU, stay on one CU in
@@ -62,6 +64,9 @@ __device__ __forceinline__ float ex(float d) { return exp2f(d * kL2E); }
 __device__ __forceinline__ float exs(float d) { return __builtin_amdgcn_exp2f(d * kL2E); }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// The same starting at any float: 16-byte accesses at 4-byte addresses cost 1-4%
+// of a streaming copy's rate (MI355X), a quarter of what scalar accesses cost.
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
 
 // Row-segment loads / stores of VW floats; NT (nontemporal) is a template
 // parameter because a runtime choice compiles to plain accesses only: the
@@ -71,8 +76,8 @@ template <int VW, bool NT>
 __device__ __forceinline__ void vld(float (&v)[VW], const float* p) {
     if constexpr (VW == 4) {
         f32x4 t;
-        if constexpr (NT) t = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
-        else t = *reinterpret_cast<const f32x4*>(p);
+        if constexpr (NT) t = __builtin_nontemporal_load(reinterpret_cast<const f32x4_any*>(p));
+        else t = *reinterpret_cast<const f32x4_any*>(p);
         v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
     } else {
         if constexpr (NT) v[0] = __builtin_nontemporal_load(p);
@@ -84,8 +89,8 @@ template <int VW, bool NT>
 __device__ __forceinline__ void vst(float* p, const float (&v)[VW]) {
     if constexpr (VW == 4) {
         const f32x4 t = {v[0], v[1], v[2], v[3]};
-        if constexpr (NT) __builtin_nontemporal_store(t, reinterpret_cast<f32x4*>(p));
-        else *reinterpret_cast<f32x4*>(p) = t;
+        if constexpr (NT) __builtin_nontemporal_store(t, reinterpret_cast<f32x4_any*>(p));
+        else *reinterpret_cast<f32x4_any*>(p) = t;
     } else {
         if constexpr (NT) __builtin_nontemporal_store(v[0], p);
         else *p = v[0];
@@ -191,9 +196,10 @@ struct SmxArgs {
 // Register-resident rows: G lanes per row, each lane holds V vectors of VW
 // floats (vector j of lane l covers elements (j*G + l)*VW ...).  Read once,
 // write once.  G <= 256: 256-thread workgroups holding 256/G rows; G > 256:
-// one row per G-thread workgroup.
+// one row per G-thread workgroup.  RAG: rows whose length is no multiple of VW;
+// the row's last vector is then read and written element by element.
 // ---------------------------------------------------------------------------
-template <int MODE, int G, int V, int VW, bool NT>
+template <int MODE, int G, int V, int VW, bool NT, bool RAG>
 __global__ __launch_bounds__(G > 256 ? G : 256) void k_smx_rows(SmxArgs p) {
     constexpr int BLK = G > 256 ? G : 256;
     constexpr int RPB = BLK / G;
@@ -212,14 +218,15 @@ __global__ __launch_bounds__(G > 256 ? G : 256) void k_smx_rows(SmxArgs p) {
 #pragma unroll
     for (int j = 0; j < V; ++j) {
         const long long e = ((long long)j * G + lane) * VW;
-        if (live && e < p.n) {
+        if (live && e + (RAG ? VW - 1 : 0) < p.n) {
             vld<VW, NT>(a[j], pa + e);
             if constexpr (BW) vld<VW, NT>(b[j], pb + e);
         } else {
 #pragma unroll
             for (int c = 0; c < VW; ++c) {
-                a[j][c] = BW ? 0.0f : -INFINITY;
-                if constexpr (BW) b[j][c] = 0.0f;
+                const bool in = RAG && live && e + c < p.n;
+                a[j][c] = in ? pa[e + c] : BW ? 0.0f : -INFINITY;
+                if constexpr (BW) b[j][c] = in ? pb[e + c] : 0.0f;
             }
         }
     }
@@ -264,7 +271,13 @@ __global__ __launch_bounds__(G > 256 ? G : 256) void k_smx_rows(SmxArgs p) {
             float o[VW];
 #pragma unroll
             for (int c = 0; c < VW; ++c) o[c] = outv<MODE>(a[j][c], BW ? b[j][c] : 0.0f, st0, st1);
-            vst<VW, NT>(po + e, o);
+            if (!RAG || e + VW <= p.n) {
+                vst<VW, NT>(po + e, o);
+            } else {
+#pragma unroll
+                for (int c = 0; c < VW - 1; ++c)
+                    if (e + c < p.n) po[e + c] = o[c];
+            }
         }
     }
 }
@@ -672,6 +685,11 @@ __global__ __launch_bounds__(PT) void k_smx_bwd_pieces(SmxArgs p, int ns, int pv
         else return (x.x * y.x + x.y * y.y) + (x.z * y.z + x.w * y.w);
     };
     const __amdgpu_buffer_rsrc_t bg = rsrc(ra, pc), by = rsrc(rb, pc);
+    // the row's last n % 4 elements: one each for the first lanes of the last piece
+    const int tail = (int)(p.n & 3);
+    const bool own_tail = pc == ns - 1 && t < tail;
+    const float tg = own_tail ? ra[4ll * q + t] : 0.0f, ty = own_tail ? rb[4ll * q + t] : 0.0f;
+    auto td = [](float x, float z) { return MODE == BWD_LOG ? x : x * z; };
     f32x4 g[kPcVR], y[kPcVR];
 #pragma unroll
     for (int j = 0; j < kPcVR; ++j) g[j] = __builtin_amdgcn_raw_buffer_load_b128(bg, (j * PT + t) * 16, 0, aux);
@@ -680,6 +698,7 @@ __global__ __launch_bounds__(PT) void k_smx_bwd_pieces(SmxArgs p, int ns, int pv
     float s = 0.0f;  // vectors past the piece read 0 (buffer range check) and add nothing
 #pragma unroll
     for (int j = 0; j < kPcVR; ++j) s += vd(g[j], y[j]);
+    s += td(tg, ty);
     s = grp<PT, false>(s, sh);
     if (t == 0) {
         parts[pc] = s;
@@ -714,12 +733,13 @@ __global__ __launch_bounds__(PT) void k_smx_bwd_pieces(SmxArgs p, int ns, int pv
         if (!((miss >> i) & 1u)) continue;  // uniform
         const __amdgpu_buffer_rsrc_t mg = rsrc(ra, i), my = rsrc(rb, i);
         float s2 = 0.0f;
-#pragma unroll
+#pragma unroll 1  // g and y stay in registers: unrolled, these loads spilled them
         for (int j = 0; j < kPcVR; ++j) {
             const f32x4 gm = __builtin_amdgcn_raw_buffer_load_b128(mg, (j * PT + t) * 16, 0, 0);
             if constexpr (MODE == BWD_LOG) s2 += vd(gm, gm);
             else s2 += vd(gm, __builtin_amdgcn_raw_buffer_load_b128(my, (j * PT + t) * 16, 0, 0));
         }
+        s2 += (i == ns - 1 && t < tail) ? td(ra[4ll * q + t], rb[4ll * q + t]) : 0.0f;
         s2 = grp<PT, false>(s2, sh);
         if (t == 0) parts[i] = s2;
         __syncthreads();
@@ -733,6 +753,7 @@ __global__ __launch_bounds__(PT) void k_smx_bwd_pieces(SmxArgs p, int ns, int pv
                          outv<MODE>(g[j].z, y[j].z, dot, 0.0f), outv<MODE>(g[j].w, y[j].w, dot, 0.0f)};
         __builtin_amdgcn_raw_buffer_store_b128(r, bo, (j * PT + t) * 16, 0, aux);  // past the piece: dropped
     }
+    if (own_tail) p.out[row * p.n + 4ll * q + t] = outv<MODE>(tg, ty, dot, 0.0f);
 }
 
 // ---------------------------------------------------------------------------
@@ -753,8 +774,9 @@ __global__ __launch_bounds__(PT) void k_smx_bwd_pieces(SmxArgs p, int ns, int pv
 // kPcVR, which the caller has set to -inf past nv.  The two give the same
 // bits: a -inf vector leaves the max alone and adds exp2(-inf) = +0 to a sum
 // that starts at +0.
+// xt: the lane's element past the row's last whole vector (-inf: none).
 template <int PT, int kPcVR, bool STREAM, class V>
-__device__ __forceinline__ void piece_stats(V&& vec, int nv, float (&sh)[2][PT / kWave], float& m, float& s) {
+__device__ __forceinline__ void piece_stats(V&& vec, float xt, int nv, float (&sh)[2][PT / kWave], float& m, float& s) {
     const f32x4 ninf = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
     (void)ninf;
     auto at = [&](int j) -> f32x4 { return vec(j); };  // held vectors: -inf past nv already
@@ -767,6 +789,7 @@ __device__ __forceinline__ void piece_stats(V&& vec, int nv, float (&sh)[2][PT /
             gm = fmaxf(fmaxf(gm, fmaxf(x.x, x.y)), fmaxf(x.z, x.w));
         }
     }
+    gm = fmaxf(gm, xt);
     float gs = 0.0f;
     if (gm != -INFINITY) {
 #pragma unroll
@@ -776,7 +799,9 @@ __device__ __forceinline__ void piece_stats(V&& vec, int nv, float (&sh)[2][PT /
                 gs += (exs(x.x - gm) + exs(x.y - gm)) + (exs(x.z - gm) + exs(x.w - gm));
             }
         }
+        gs += exs(xt - gm);
     } else {
+        gs += xt != xt ? xt : 0.0f;
 #pragma unroll
         for (int j = 0; j < (STREAM ? 1 : kPcVR); ++j) {
             for (int jj = j; jj < (STREAM ? n : j + 1); ++jj) {  // only -inf and NaN: NaN stays
@@ -833,7 +858,10 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 #pragma unroll
         for (int j = 0; j < kPcVR; ++j) x[j] = j < nv ? x[j] : ninf;
     }
-    piece_stats<PT, kPcVR, false>([&](int j) { return x[j]; }, kPcVR, sh, m, s);
+    const int tail = (int)(p.n & 3);
+    const bool own_tail = pc == ns - 1 && t < tail;
+    const float xt = own_tail ? ra[4ll * q + t] : -INFINITY;
+    piece_stats<PT, kPcVR, false>([&](int j) { return x[j]; }, xt, kPcVR, sh, m, s);
     if (t == 0) {
         pm[pc] = m;
         ps[pc] = s;
@@ -874,8 +902,8 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(4, 8))) void
         const __amdgpu_buffer_rsrc_t mx = rsrc(ra, i);
         float m2, s2;
         piece_stats<PT, kPcVR, true>(
-            [&](int j) { return __builtin_amdgcn_raw_buffer_load_b128(mx, (j * PT + t) * 16, 0, 0); }, nv_of(i), sh,
-            m2, s2);
+            [&](int j) { return __builtin_amdgcn_raw_buffer_load_b128(mx, (j * PT + t) * 16, 0, 0); },
+            i == ns - 1 && t < tail ? ra[4ll * q + t] : -INFINITY, nv_of(i), sh, m2, s2);
         if (t == 0) {
             pm[i] = m2;
             ps[i] = s2;
@@ -900,6 +928,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(4, 8))) void
                          outv<MODE>(x[j].z, 0.0f, st0, st1), outv<MODE>(x[j].w, 0.0f, st0, st1)};
         __builtin_amdgcn_raw_buffer_store_b128(r, bo, (j * PT + t) * 16, 0, aux);  // past the piece: dropped
     }
+    if (own_tail) ro[4ll * q + t] = outv<MODE>(xt, 0.0f, st0, st1);
 }
 
 // ---------------------------------------------------------------------------
@@ -1691,68 +1720,69 @@ int run_f64(const SmxF64Args& a, hipStream_t st) {
 // ---------------------------------------------------------------------------
 // Host planner
 // ---------------------------------------------------------------------------
-template <int MODE, int G, int V, int VW>
+// Whether launches on the stream are being recorded into a graph.
+bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
+        (void)hipGetLastError();  // not an error of this call
+        return true;
+    }
+    return cs != hipStreamCaptureStatusNone;
+}
+
+template <int MODE, int G, int V>
 int launch_rows(const SmxArgs& a, hipStream_t st) {
     constexpr int BLK = G > 256 ? G : 256;
     constexpr int RPB = BLK / G;
-    const long long blocks = (a.rows + RPB - 1) / RPB;
-    if (a.nt) hipLaunchKernelGGL((k_smx_rows<MODE, G, V, VW, true>), dim3((unsigned)blocks), dim3(BLK), 0, st, a);
-    else hipLaunchKernelGGL((k_smx_rows<MODE, G, V, VW, false>), dim3((unsigned)blocks), dim3(BLK), 0, st, a);
+    const dim3 blocks((unsigned)((a.rows + RPB - 1) / RPB)), blk(BLK);
+    if (a.n % 4) {
+        if (a.nt) hipLaunchKernelGGL((k_smx_rows<MODE, G, V, 4, true, true>), blocks, blk, 0, st, a);
+        else hipLaunchKernelGGL((k_smx_rows<MODE, G, V, 4, false, true>), blocks, blk, 0, st, a);
+    } else {
+        if (a.nt) hipLaunchKernelGGL((k_smx_rows<MODE, G, V, 4, true, false>), blocks, blk, 0, st, a);
+        else hipLaunchKernelGGL((k_smx_rows<MODE, G, V, 4, false, false>), blocks, blk, 0, st, a);
+    }
     return check_launch("tpr_softmax (rows)");
 }
 
-// Single-pass variants: VW = 4 -> G in {16, 64, 256, 1024}, V in {1, 2, 4, 8},
-// and forward rows of 16385..32768 floats on 512 lanes with V = 16 (two
-// workgroups per CU, so one loads while the other reduces: 67% vs 55% of the
-// HBM peak with one 1024-lane workgroup per CU); VW = 1 -> G in {64, 256, 1024},
-// V in {4, 16} (backward: 4).  Returns -1 when the row is too long.
+// Single-pass variants: G in {16, 64, 256, 1024}, V in {1, 2, 4, 8}, and forward
+// rows of 16385..32768 floats on 512 lanes with V = 16 (two workgroups per CU,
+// so one loads while the other reduces: 67% vs 55% of the HBM peak with one
+// 1024-lane workgroup per CU).  Rows start and end at any float (MI355X, us,
+// scalar -> vector: softmax [100000, 77] 20.1 -> 11.4, [8192, 769] 10.7 -> 9.7,
+// its gradient at [37, 4099] 7.9 -> 3.8).
+// Returns -1 when the row is too long.
 template <int MODE>
-int rows_single(const SmxArgs& a, int vw, hipStream_t st) {
+int rows_single(const SmxArgs& a, hipStream_t st) {
     constexpr bool BW = MODE >= BWD;
-    const long long n = a.n;
-    if (vw == 4) {
-        const long long q = (n + 3) / 4;  // vectors per row
-        const int vmax = 8;
-        auto pick = [&](int g) -> int {  // smallest V with g*V >= q, or 0
-            for (int v = 1; v <= vmax; v *= 2)
-                if ((long long)g * v >= q) return v;
-            return 0;
-        };
-        // fewest lanes that keep V <= 4, else the widest workgroup with V = 8
-        if constexpr (!BW) {
-            if (knobs().smx_lanes != 1024 && q > 4096 && q <= 8192) return launch_rows<MODE, 512, 16, 4>(a, st);
-        }
-        for (int g : {16, 64, 256, 1024}) {
-            const int v = pick(g);
-            if (v == 0 || (v > 4 && g < 1024)) continue;
+    const long long q = (a.n + 3) / 4;  // vectors per row
+    const int vmax = 8;
+    auto pick = [&](int g) -> int {  // smallest V with g*V >= q, or 0
+        for (int v = 1; v <= vmax; v *= 2)
+            if ((long long)g * v >= q) return v;
+        return 0;
+    };
+    // fewest lanes that keep V <= 4, else the widest workgroup with V = 8
+    if constexpr (!BW) {
+        if (knobs().smx_lanes != 1024 && q > 4096 && q <= 8192) return launch_rows<MODE, 512, 16>(a, st);
+    }
+    for (int g : {16, 64, 256, 1024}) {
+        const int v = pick(g);
+        if (v == 0 || (v > 4 && g < 1024)) continue;
 #define TPR_SMX_V(GG)                                                              \
     switch (v) {                                                                   \
-        case 1: return launch_rows<MODE, GG, 1, 4>(a, st);                         \
-        case 2: return launch_rows<MODE, GG, 2, 4>(a, st);                         \
-        case 4: return launch_rows<MODE, GG, 4, 4>(a, st);                         \
-        default: return launch_rows<MODE, GG, 8, 4>(a, st);                        \
+        case 1: return launch_rows<MODE, GG, 1>(a, st);                            \
+        case 2: return launch_rows<MODE, GG, 2>(a, st);                            \
+        case 4: return launch_rows<MODE, GG, 4>(a, st);                            \
+        default: return launch_rows<MODE, GG, 8>(a, st);                           \
     }
-            switch (g) {
-                case 16: TPR_SMX_V(16)
-                case 64: TPR_SMX_V(64)
-                case 256: TPR_SMX_V(256)
-                default: TPR_SMX_V(1024)
-            }
+        switch (g) {
+            case 16: TPR_SMX_V(16)
+            case 64: TPR_SMX_V(64)
+            case 256: TPR_SMX_V(256)
+            default: TPR_SMX_V(1024)
+        }
 #undef TPR_SMX_V
-        }
-        return -1;
-    }
-    for (int g : {64, 256, 1024}) {
-        if ((long long)g * 4 >= n) {
-            switch (g) {
-                case 64: return launch_rows<MODE, 64, 4, 1>(a, st);
-                case 256: return launch_rows<MODE, 256, 4, 1>(a, st);
-                default: return launch_rows<MODE, 1024, 4, 1>(a, st);
-            }
-        }
-    }
-    if constexpr (!BW) {
-        if (n <= 1024LL * 16) return launch_rows<MODE, 1024, 16, 1>(a, st);
     }
     return -1;
 }
@@ -1816,11 +1846,12 @@ int launch_res(const SmxArgs& a, int vr, hipStream_t st) {
 #undef TPR_RES
 }
 
-// Pieces per row for k_smx_bwd_pieces with PT-thread workgroups (0: not
-// taken): softmax gradients of rows of 16384 .. kPcMax * PT * kPcVR * 4
-// floats, 16-byte vectors.
-int bwd_pieces(long long n, int vw, int pt, int vr) {
-    if (vw != 4 || n <= 16384 || knobs().smx_pieces < 0 || knobs().smx_two_pass) return 0;
+// Pieces per row of the piece kernels with pt-thread workgroups holding vr float4
+// per lane (0: not taken): rows of 16385 .. kPcMax * pt * vr * 4 floats, starting
+// and ending at any float.  Not under graph capture: a replayed launch carries
+// the tag of its capture, so a replay could take the partials of the one before.
+int row_pieces(long long n, int pt, int vr, hipStream_t st) {
+    if (n <= 16384 || knobs().smx_pieces < 0 || knobs().smx_two_pass || capturing(st)) return 0;
     const long long q = n / 4;
     const long long per = (long long)pt * vr;
     const long long ns = (q + per - 1) / per;
@@ -1874,7 +1905,7 @@ int run_rows(const SmxArgs& a0, int vw, hipStream_t st) {
         // [1024, 32768] 67.2 against 74.2 (g held)
         // (one slot per piece: a launch whose pieces outnumber the slots would
         // reuse a slot under the same epoch, so it takes the kernels below)
-        const int ns = bwd_pieces(a.n, vw, 512, 24);
+        const int ns = row_pieces(a.n, 512, 24, st);
         if (ns > 0 && a.rows * ns <= kSmxSlots) return launch_bwd_pieces<MODE, 512, 24>(a, ns, st);
     } else if (knobs().smx_fwd_pieces >= 0) {
         // forward: x held by row pieces when the one-row-per-CU kernel below
@@ -1886,11 +1917,15 @@ int run_rows(const SmxArgs& a0, int vw, hipStream_t st) {
         // and [1024, 32768] (one piece per row) 43.9 -> 48.3.  Rows longer than
         // one CU holds (> 153600 floats) take them at any row count instead of
         // streaming twice: [64, 262144] 44.4 -> 28.6, [32, 500000] 45.9 ->
-        // 33.9, [512, 163840] 153 -> 120, [8, 655360] 25.0 -> 20.8.  The test
+        // 33.9, [512, 163840] 153 -> 120, [8, 655360] 25.0 -> 20.8.  Rows that do
+        // not start and end on 16 bytes (vw = 1) always take them: the resident
+        // kernel's LDS loads need aligned rows, and the kernels below read such
+        // rows twice, float by float ([2048, 50257] 234 -> 155, its gradient 347
+        // -> 237, log 230 -> 150 and 309 -> 225).  The test
         // knob smx_fwd_pieces = 1 takes every row the pieces can hold.
-        const int ns = bwd_pieces(a.n, vw, 512, kFwdPcVR);
+        const int ns = row_pieces(a.n, 512, kFwdPcVR, st);
         if (ns > 0 && a.rows * ns * 2 <= kSmxSlots &&  // two slots per piece, none reused in a launch
-            (knobs().smx_fwd_pieces > 0 || (ns >= 2 && a.rows > device_info().cus) ||
+            (knobs().smx_fwd_pieces > 0 || vw != 4 || (ns >= 2 && a.rows > device_info().cus) ||
              (a.n > kResMax && knobs().smx_fwd_pieces == 0)))
             return launch_fwd_pieces<MODE, 512, kFwdPcVR>(a, ns, st);
     }
@@ -1907,7 +1942,7 @@ int run_rows(const SmxArgs& a0, int vw, hipStream_t st) {
         return launch_res<MODE>(a, vr, st);
     }
     if (!two_pass) {
-        const int rc = rows_single<MODE>(a, vw, st);
+        const int rc = rows_single<MODE>(a, st);
         if (rc >= 0) return rc;
     }
     constexpr bool BW = MODE >= BWD;
@@ -1950,7 +1985,7 @@ int run_cols(const SmxColArgs& a, hipStream_t st) {
             if constexpr (!BW) {
                 const long long gp = 2 * blocks;
                 if (a.n > 512 && a.n <= 1024 && knobs().smx_res >= 0 && knobs().smx_two_pass == 0 &&
-                    knobs().smx_fwd_pieces >= 0 && knobs().smx_pieces >= 0 && gp * 128 <= kSmxSlots) {
+                    knobs().smx_fwd_pieces >= 0 && knobs().smx_pieces >= 0 && gp * 128 <= kSmxSlots && !capturing(st)) {
                     unsigned ep = smx_epoch_ctr.fetch_add(1, std::memory_order_relaxed) + 1u;
                     if (ep == 0) ep = smx_epoch_ctr.fetch_add(1, std::memory_order_relaxed) + 1u;
                     const int spin = knobs().smx_spin < 0 ? 0 : 4000;
