@@ -25,9 +25,11 @@ namespace tpr {
 namespace {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef f32x4_t f32x4_any __attribute__((aligned(4)));  // outputs start at any float
 
 constexpr int kNllBlock = 256;
 constexpr int kNllMaxBlocks = 1024;
+constexpr long long kNllOne = 4096;  // most samples of the single-workgroup forward
 
 struct NllPart {
     double loss;
@@ -54,13 +56,34 @@ __device__ __forceinline__ T wave_sum(T v) {
     return v;
 }
 
-__global__ __launch_bounds__(kNllBlock) void k_nll_part(NllArgs a) {
-    __shared__ double sl[kNllBlock / kWave], sw[kNllBlock / kWave];
-    __shared__ int sb[kNllBlock / kWave];
+struct NllFin {
+    const NllPart* part;
+    int nparts;
+    long long reduction;
+    float* out;
+    float* total_weight;
+    int* status;
+};
+
+__device__ __forceinline__ void nll_finish(const NllFin& f, const NllPart& p) {
+    double l = p.loss;
+    const float tw = (float)p.weight;
+    if (f.reduction == 1 && tw > 0.0f) l /= (double)tw;
+    if (f.reduction != 0) f.out[0] = (float)l;
+    f.total_weight[0] = tw;
+    if (f.status) f.status[0] = p.bad;
+}
+
+// BLK threads per workgroup.  ONE: a single workgroup takes all samples and
+// finishes the sums itself (up to kNllOne samples: four per thread), instead of
+// a second launch over the workgroups' partial sums.
+template <int BLK, bool ONE>
+__global__ __launch_bounds__(BLK) void k_nll_part(NllArgs a, NllFin f) {
+    __shared__ double sl[BLK / kWave], sw[BLK / kWave];
+    __shared__ int sb[BLK / kWave];
     double loss = 0.0, wsum = 0.0;
     int bad = 0;
-    for (long long i = (long long)blockIdx.x * kNllBlock + threadIdx.x; i < a.n;
-         i += (long long)gridDim.x * kNllBlock) {
+    for (long long i = (long long)blockIdx.x * BLK + threadIdx.x; i < a.n; i += (long long)gridDim.x * BLK) {
         const long long t = a.t[i * a.ts];
         float li = 0.0f;
         if (t != a.ignore) {
@@ -87,23 +110,15 @@ __global__ __launch_bounds__(kNllBlock) void k_nll_part(NllArgs a) {
     __syncthreads();
     if (threadIdx.x == 0) {
         NllPart p{0.0, 0.0, 0, 0};
-        for (int k = 0; k < kNllBlock / kWave; ++k) {
+        for (int k = 0; k < BLK / kWave; ++k) {
             p.loss += sl[k];
             p.weight += sw[k];
             p.bad |= sb[k] != 0;
         }
-        a.part[blockIdx.x] = p;
+        if constexpr (ONE) nll_finish(f, p);
+        else a.part[blockIdx.x] = p;
     }
 }
-
-struct NllFin {
-    const NllPart* part;
-    int nparts;
-    long long reduction;
-    float* out;
-    float* total_weight;
-    int* status;
-};
 
 __global__ __launch_bounds__(kNllBlock) void k_nll_fin(NllFin f) {
     __shared__ double sl[kNllBlock / kWave], sw[kNllBlock / kWave];
@@ -126,18 +141,13 @@ __global__ __launch_bounds__(kNllBlock) void k_nll_fin(NllFin f) {
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        double l = 0.0, ws = 0.0;
-        int b = 0;
+        NllPart p{0.0, 0.0, 0, 0};
         for (int k = 0; k < kNllBlock / kWave; ++k) {
-            l += sl[k];
-            ws += sw[k];
-            b |= sb[k] != 0;
+            p.loss += sl[k];
+            p.weight += sw[k];
+            p.bad |= sb[k] != 0;
         }
-        const float tw = (float)ws;
-        if (f.reduction == 1 && tw > 0.0f) l /= (double)tw;
-        if (f.reduction != 0) f.out[0] = (float)l;
-        f.total_weight[0] = tw;
-        if (f.status) f.status[0] = b;
+        nll_finish(f, p);
     }
 }
 
@@ -151,7 +161,6 @@ struct NllBwdArgs {
     const float* tw;
     long long n, c, reduction, ignore;
     float* gi;
-    long long chunks;  // workgroups per row (row kernel)
 };
 
 __device__ __forceinline__ float nll_grad_value(const NllBwdArgs& a, long long i, long long t) {
@@ -164,38 +173,70 @@ __device__ __forceinline__ float nll_grad_value(const NllBwdArgs& a, long long i
     return -w * g;
 }
 
-// Rows of at least 1024 elements: workgroup (row, chunk) writes 256 * kNllU
-// 16-byte vectors (VW = 4) or scalars (VW = 1) of one row.
-// Vectors each thread of the row kernel writes: one (a write-only kernel runs
-// fastest with one 16-byte store per thread over a grid covering the output:
-// measured on MI355X, a 256 MiB fill takes 40 us against 45-52 us with 2-8
-// stores per thread).
-constexpr int kNllU = 1;
-
-template <int VW>
-__global__ __launch_bounds__(kNllBlock) void k_nll_bwd_rows(NllBwdArgs a) {
-    constexpr long long CH = (long long)kNllBlock * kNllU * VW;
-    const long long row = blockIdx.x / a.chunks;
-    const long long base = (blockIdx.x - row * a.chunks) * CH;
-    const long long t = a.t[row * a.ts];
-    const bool hit = t != a.ignore && t >= 0 && t < a.c;
-    const float v = hit ? nll_grad_value(a, row, t) : 0.0f;
-    float* out = a.gi + row * a.c;
-#pragma unroll
-    for (int u = 0; u < kNllU; ++u) {
-        const long long e = base + ((long long)u * kNllBlock + threadIdx.x) * VW;
-        if (e >= a.c) break;
-        if constexpr (VW == 4) {
-            f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (hit && t >= e && t < e + 4) z[t - e] = v;
-            __builtin_nontemporal_store(z, reinterpret_cast<f32x4_t*>(out + e));
-        } else {
-            __builtin_nontemporal_store((hit && t == e) ? v : 0.0f, out + e);
-        }
+// The dense [n, c] gradient is written as one flat run, one 16-byte store per
+// thread (a write-only kernel runs fastest that way over a grid covering the
+// output: measured on MI355X, a 256 MiB fill takes 40 us against 45-52 us with
+// 2-8 stores per thread), so stores stay on 16 bytes whatever c is and a vector
+// may hold the end of one row and the start of the next.  [4096, 50257]: one
+// scalar store per thread took 377 us, vectors row by row (any alignment) 171,
+// this 113 (7.3 TB/s); [4096, 32000] 78 -> 73.
+__device__ __forceinline__ void nll_store(float* out, long long e, long long total, f32x4_t z) {
+    if (e + 4 <= total) {
+        __builtin_nontemporal_store(z, reinterpret_cast<f32x4_any*>(out + e));
+    } else {
+        for (int k = 0; e + k < total; ++k) out[e + k] = z[k];
     }
 }
 
-// Short rows: one element per thread over the flat [n, c] output.
+// Rows of at least 1024 elements: the 1024 elements of a workgroup lie in two
+// rows at most.
+__global__ __launch_bounds__(kNllBlock) void k_nll_bwd_rows(NllBwdArgs a) {
+    const long long base = (long long)blockIdx.x * (4 * kNllBlock);
+    const long long row = base / a.c;
+    const long long col = base - row * a.c + 4 * threadIdx.x;  // may pass the row's end
+    const long long total = a.n * a.c;
+    if (base + 4 * threadIdx.x >= total) return;
+    long long t0 = a.t[row * a.ts];
+    if (t0 == a.ignore || t0 < 0 || t0 >= a.c) t0 = -4;
+    long long t1 = row + 1 < a.n ? a.t[(row + 1) * a.ts] : a.ignore;
+    t1 = (t1 == a.ignore || t1 < 0 || t1 >= a.c) ? -4 : t1 + a.c;
+    f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (t0 >= col && t0 < col + 4) {
+        const float v = nll_grad_value(a, row, t0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) z[k] = t0 == col + k ? v : z[k];
+    }
+    if (t1 >= col && t1 < col + 4) {
+        const float v = nll_grad_value(a, row + 1, t1 - a.c);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) z[k] = t1 == col + k ? v : z[k];
+    }
+    nll_store(a.gi, base + 4 * threadIdx.x, total, z);
+}
+
+// Shorter rows (n * c < 2^32 - 1024): one 32-bit division per vector.  [8192,
+// 1000]: one element per thread with a 64-bit division each took 12.7 us, this
+// this 6.7 us.
+__global__ __launch_bounds__(kNllBlock) void k_nll_bwd_short(NllBwdArgs a) {
+    const unsigned e = (blockIdx.x * (unsigned)kNllBlock + threadIdx.x) * 4u;
+    const unsigned c = (unsigned)a.c, total = (unsigned)(a.n * a.c);
+    if (e >= total) return;
+    unsigned row = e / c, col = e - row * c;
+    long long t = a.t[(long long)row * a.ts];
+    f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (t == (long long)col && t != a.ignore) z[k] = nll_grad_value(a, row, t);
+        if (++col == c && e + k + 1 < total) {
+            col = 0;
+            t = a.t[(long long)++row * a.ts];
+        }
+    }
+    nll_store(a.gi, e, total, z);
+}
+
+// Short rows beyond 32-bit indices: one element per thread over the
+// flat [n, c] output.
 __global__ __launch_bounds__(kNllBlock) void k_nll_bwd_flat(NllBwdArgs a) {
     const long long total = a.n * a.c;
     for (long long e = (long long)blockIdx.x * kNllBlock + threadIdx.x; e < total;
@@ -241,11 +282,15 @@ extern "C" int tpr_nll_loss(const void* input, int32_t dtype, int64_t n, int64_t
     NllArgs a{static_cast<const float*>(input), n, c, s0, s1,
               reinterpret_cast<const long long*>(target), ts, static_cast<const float*>(weight),
               reduction, ignore_index, static_cast<float*>(out), part};
-    hipLaunchKernelGGL(k_nll_part, dim3((unsigned)blocks), dim3(kNllBlock), 0, st, a);
-    int rc = check_launch("tpr_nll_loss");
-    if (rc) return rc;
     NllFin f{part, (int)blocks, reduction, static_cast<float*>(out), static_cast<float*>(total_weight),
              reinterpret_cast<int*>(status)};
+    if (n <= kNllOne) {
+        hipLaunchKernelGGL((k_nll_part<1024, true>), dim3(1), dim3(1024), 0, st, a, f);
+        return check_launch("tpr_nll_loss");
+    }
+    hipLaunchKernelGGL((k_nll_part<kNllBlock, false>), dim3((unsigned)blocks), dim3(kNllBlock), 0, st, a, f);
+    int rc = check_launch("tpr_nll_loss");
+    if (rc) return rc;
     hipLaunchKernelGGL(k_nll_fin, dim3(1), dim3(kNllBlock), 0, st, f);
     return check_launch("tpr_nll_loss (finalize)");
 }
@@ -262,15 +307,14 @@ extern "C" int tpr_nll_loss_backward(const void* grad_output, int64_t gs, const 
     hipStream_t st = static_cast<hipStream_t>(stream);
     NllBwdArgs a{static_cast<const float*>(grad_output), gs, reinterpret_cast<const long long*>(target), ts,
                  static_cast<const float*>(weight), static_cast<const float*>(total_weight),
-                 n, c, reduction, ignore_index, static_cast<float*>(grad_input), 0};
+                 n, c, reduction, ignore_index, static_cast<float*>(grad_input)};
     if (c >= 1024) {
-        const bool v4 = c % 4 == 0 && (reinterpret_cast<uintptr_t>(grad_input) & 15) == 0;
-        const long long ch = (long long)kNllBlock * kNllU * (v4 ? 4 : 1);
-        a.chunks = (c + ch - 1) / ch;
-        const long long blocks = n * a.chunks;
+        const long long blocks = (n * c + 4 * kNllBlock - 1) / (4 * kNllBlock);
         if (blocks > 0x7fffffffLL) return fail(TPR_ERR_INVALID_ARG, "tpr_nll_loss_backward: too large");
-        if (v4) hipLaunchKernelGGL((k_nll_bwd_rows<4>), dim3((unsigned)blocks), dim3(kNllBlock), 0, st, a);
-        else hipLaunchKernelGGL((k_nll_bwd_rows<1>), dim3((unsigned)blocks), dim3(kNllBlock), 0, st, a);
+        hipLaunchKernelGGL(k_nll_bwd_rows, dim3((unsigned)blocks), dim3(kNllBlock), 0, st, a);
+    } else if (n * c < 0x100000000LL - 4 * kNllBlock) {
+        const unsigned blocks = (unsigned)((n * c + 4 * kNllBlock - 1) / (4 * kNllBlock));
+        hipLaunchKernelGGL(k_nll_bwd_short, dim3(blocks), dim3(kNllBlock), 0, st, a);
     } else {
         long long blocks = (n * c + kNllBlock - 1) / kNllBlock;
         const long long cap = (long long)device_info().cus * 32;
