@@ -396,14 +396,21 @@ __device__ void split_finish(typename Op::State st, typename Op::State* part, un
     }
 }
 
-// Streaming 128-bit load; `nt` marks it nontemporal (read once, do not keep in cache).
+// Streaming 128-bit load at any float; `nt` marks it nontemporal (read once, do
+// not keep in cache).  16-byte loads at 4-byte addresses cost 1-2% of a
+// streaming read's rate (MI355X).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ float4 ld4(const float4* p, int nt) {
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+__device__ __forceinline__ float4 ld4(const float* p, int nt) {
     if (nt) {
-        const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
+        const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_any*>(p));
         return make_float4(v.x, v.y, v.z, v.w);
     }
-    return *p;
+    // not the same vector type: the compiler would merge the two branches' loads
+    // into one and drop the nontemporal mark (C4 sum 153 -> 170 us)
+    unsigned __int128 w;
+    __builtin_memcpy(&w, p, 16);
+    return __builtin_bit_cast(float4, w);
 }
 
 template <class Op, class I>
@@ -441,15 +448,19 @@ struct RowArgs {
     unsigned* tickets;  // S > 1, one row per workgroup: per-row counters of split_finish (else null)
 };
 
-template <class Op, int VEC, int LANES, int U>
+template <class Op>
+constexpr bool kHeavyAcc = std::is_same<Op, NormOp<0>>::value;  // powf
+
+template <class Op, int LANES, int U>
 __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void k_rows(RowArgs a) {
     using Acc = typename Op::Acc;
-    using State = typename Op::State;
+    using Final = typename Finish<Op>::Final;
+    using State = typename Final::State;
     constexpr int BLK = LANES > kBlock ? LANES : kBlock;  // one long row per 512/1024-thread block
     constexpr int GROUPS = (LANES >= BLK) ? 1 : BLK / LANES;
     // U = vectors in flight per lane
     constexpr int TILE = U * LANES;       // vectors per tile (contiguous in memory)
-    const float prm = a.fin.p;            // op parameter (NORM exponent)
+    float prm = a.fin.p;                  // op parameter (NORM exponent; var / std: the row's shift)
     const int tid = threadIdx.x;
     const int g = tid / LANES;
     const int l = tid % LANES;
@@ -468,17 +479,55 @@ __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void k_rows(RowArg
     if (row < a.rows) {
         const float* p = a.in + row * a.row_stride;
         const int step = a.S * TILE;
-        if (VEC == 4) {
-            const int nv = (int)(a.R >> 2);
-            const float4* pv = reinterpret_cast<const float4*>(p);
-            int t0 = s * TILE;
-            for (; t0 + TILE <= nv; t0 += step) {
-                float4 t[U];
+        // rows of a few elements (16 lanes): one element per lane and load; few
+        // lanes would hold a vector ([1000003, 7] sum 48 -> 39 us)
+        const int nv = LANES == 16 && a.R < 32 ? 0 : (int)(a.R >> 2);
+        if constexpr (LANES == 16) {
+            if (a.R < 32 && s == 0 && l < a.R) {
+                if constexpr (Finish<Op>::kShift) prm = p[0];
+                const float x0 = p[l];
+                float x1 = 0.0f;
+                if (a.R > 16) x1 = p[min(l + 16, (int)a.R - 1)];
+                Op::acc(acc, x0, l, prm);
+                if (l + 16 < a.R) Op::acc(acc, x1, l + 16, prm);
+            }
+        }
+        // the last R % 4 elements: one each for the first lanes, loaded first
+        const int te = 4 * nv + l;
+        const bool tail = s == 0 && te < a.R && !(LANES == 16 && a.R < 32);
+        float xt = 0.0f;
+        if (tail) xt = p[te];
+        if constexpr (Finish<Op>::kShift) prm = p[0];  // a row has at least one element
+        int t0 = s * TILE;
+        for (; t0 + TILE <= nv; t0 += step) {
+            float4 t[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) t[u] = ld4(pv + t0 + l + u * LANES, a.nt);
+            for (int u = 0; u < U; ++u) t[u] = ld4(p + 4ll * (t0 + l + u * LANES), a.nt);
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int v = t0 + l + u * LANES;
+            for (int u = 0; u < U; ++u) {
+                const int v = t0 + l + u * LANES;
+                if constexpr (Op::kIndexed) {
+                    Op::acc(accq[0], t[u].x, v, prm);
+                    Op::acc(accq[1 % (Op::kIndexed ? 4 : 1)], t[u].y, v, prm);
+                    Op::acc(accq[2 % (Op::kIndexed ? 4 : 1)], t[u].z, v, prm);
+                    Op::acc(accq[3 % (Op::kIndexed ? 4 : 1)], t[u].w, v, prm);
+                } else {
+                    acc4<Op>(acc, t[u], 4 * v, prm);
+                }
+            }
+        }
+        if constexpr (kHeavyAcc<Op>) {  // one copy of the step: it is hundreds of instructions
+            for (int e = 4 * t0 + l; e < 4 * nv; e += LANES) Op::acc(acc, p[e], e, prm);
+        } else if (t0 < nv) {
+            // past the row's last vector: that vector again, not accumulated
+            float4 t[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (t0 + u * LANES < nv) t[u] = ld4(p + 4ll * min(t0 + l + u * LANES, nv - 1), a.nt);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int v = t0 + l + u * LANES;
+                if (v < nv) {
                     if constexpr (Op::kIndexed) {
                         Op::acc(accq[0], t[u].x, v, prm);
                         Op::acc(accq[1 % (Op::kIndexed ? 4 : 1)], t[u].y, v, prm);
@@ -489,66 +538,36 @@ __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void k_rows(RowArg
                     }
                 }
             }
-            if (t0 < nv) {
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int v = t0 + l + u * LANES;
-                    if (v < nv) {
-                        const float4 t = pv[v];
-                        if constexpr (Op::kIndexed) {
-                            Op::acc(accq[0], t.x, v, prm);
-                            Op::acc(accq[1 % (Op::kIndexed ? 4 : 1)], t.y, v, prm);
-                            Op::acc(accq[2 % (Op::kIndexed ? 4 : 1)], t.z, v, prm);
-                            Op::acc(accq[3 % (Op::kIndexed ? 4 : 1)], t.w, v, prm);
-                        } else {
-                            acc4<Op>(acc, t, 4 * v, prm);
-                        }
-                    }
-                }
-            }
-            for (int e = 4 * nv + s * LANES + l; e < a.R; e += a.S * LANES) Op::acc(acc, p[e], e, prm);
-        } else {
-            int t0 = s * TILE;
-            for (; t0 + TILE <= a.R; t0 += step) {
-                float x[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) x[u] = p[t0 + l + u * LANES];
-#pragma unroll
-                for (int u = 0; u < U; ++u) Op::acc(acc, x[u], t0 + l + u * LANES, prm);
-            }
-            if (t0 < a.R) {
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int e = t0 + l + u * LANES;
-                    if (e < a.R) Op::acc(acc, p[e], e, prm);
-                }
-            }
         }
+        if (tail) Op::acc(acc, xt, te, prm);
     }
 
-    State st = Op::state(acc);
+    typename Op::State os = Op::state(acc);
     if constexpr (Op::kIndexed) {
+        if (LANES > 16 || a.R >= 32) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) st = Op::comb(st, Op::state_scaled(accq[q % (Op::kIndexed ? 4 : 1)], 4, q));
-    }
-    constexpr int SUBW = LANES < kWave ? LANES : kWave;
-    st = group_reduce_sub_wave<Op, SUBW>(st);
-    if (LANES > kWave) {
-        constexpr int WPG = LANES / kWave;  // waves per group
-        __shared__ State sh[BLK / kWave];
-        const int w = tid / kWave;
-        if (__lane_id() == 0) sh[w] = st;
-        __syncthreads();
-        if (l == 0) {
-            State r = sh[g * WPG];
-#pragma unroll
-            for (int i = 1; i < WPG; ++i) r = Op::comb(r, sh[g * WPG + i]);
-            st = r;
+            for (int q = 0; q < 4; ++q) os = Op::comb(os, Op::state_scaled(accq[q % (Op::kIndexed ? 4 : 1)], 4, q));
         }
     }
+    constexpr int SUBW = LANES < kWave ? LANES : kWave;
+    os = group_reduce_sub_wave<Op, SUBW>(os);
+    if constexpr (LANES > kWave) {
+        constexpr int WPG = LANES / kWave;  // waves per group
+        __shared__ typename Op::State sh[BLK / kWave];
+        const int w = tid / kWave;
+        if (__lane_id() == 0) sh[w] = os;
+        __syncthreads();
+        if (l == 0) {
+            typename Op::State r = sh[g * WPG];
+#pragma unroll
+            for (int i = 1; i < WPG; ++i) r = Op::comb(r, sh[g * WPG + i]);
+            os = r;
+        }
+    }
+    const State st = Finish<Op>::of(os, prm);
     if constexpr (GROUPS == 1) {
         if (a.tickets) {
-            split_finish<Op, BLK>(st, reinterpret_cast<State*>(a.part), a.tickets + row, a.S, s, a.rows, row,
+            split_finish<Final, BLK>(st, reinterpret_cast<State*>(a.part), a.tickets + row, a.S, s, a.rows, row,
                                   [&](const State& r) { fin_write(r, a.fin, a.out, row); });
             return;
         }
@@ -561,11 +580,11 @@ __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void k_rows(RowArg
 
 // ---------------------------------------------------------------------------
 // Register-row kernel for ops whose identity is 0 (sum, mean, norm p = 1/2,
-// any): [rows, R], R contiguous, R % 4 == 0, rows 16-byte aligned,
-// R/4 <= 64*WPR*NV.  WPR waves share a row; every lane issues all of its NV
+// any): [rows, R], R contiguous, rows starting and ending at any float,
+// R <= 4*64*WPR*NV.  WPR waves share a row; every lane issues all of its NV
 // 128-bit nontemporal loads before it adds anything, so a row is one burst of
 // loads with no branch between them.  Loads go through a buffer resource whose
-// range is the row (0 for a row past the end): vectors out of range read 0
+// range is the row (0 for a row past the end): words out of range read 0
 // without touching memory, which these ops ignore.  RPB = BLK / (64*WPR) rows
 // per workgroup.  Measured on MI355X (HIP events, 256 MiB inputs): sum over
 // rows of 512-2048 floats 38.4 us against 40.1-40.6 us for k_rows; rows of
@@ -648,15 +667,17 @@ __global__ __launch_bounds__(BLK) void k_rows_reg(RowArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// var / std over rows that fill WPR waves exactly (R == 4 * 64 * WPR * NV):
+// var / std over rows of up to 4 * 64 * WPR * NV floats (FULL: exactly that many):
 // every element is shifted by the row's first element K (one scalar load per
 // wave), so the shifted sums S1 = sum(x - K), S2 = sum((x - K)^2) of all lanes
 // add up directly -- no per-lane Welford state, no Chan merges, one divide per
 // row: mean = K + S1/n, M2 = S2 - S1^2/n (fp64; K is an element of the row, the
 // same kind of shift the per-thread Welford accumulator uses).  Four chains per
-// lane (one per float4 component), all loads issued before the first add.
+// lane (one per float4 component), all loads issued before the first add; not
+// FULL: words past the row's end (the buffer's range) count as K and add 0.
+// MI355X: [64323, 1023] 49 -> 38 us against k_rows.
 // ---------------------------------------------------------------------------
-template <int NV, int WPR, int BLK>
+template <int NV, int WPR, int BLK, bool FULL>
 __global__ __launch_bounds__(BLK) void k_rows_reg_var(RowArgs a) {
     constexpr int RPB = BLK / (kWave * WPR);
     static_assert(RPB >= 1 && RPB * kWave * WPR == BLK, "BLK must hold whole rows");
@@ -678,6 +699,14 @@ __global__ __launch_bounds__(BLK) void k_rows_reg_var(RowArgs a) {
     const double Kd = (double)__uint_as_float(
         __builtin_amdgcn_readfirstlane(__builtin_amdgcn_raw_buffer_load_b32(rs, 0, 0, 0)));
     double s1[4] = {0.0, 0.0, 0.0, 0.0}, s2[4] = {0.0, 0.0, 0.0, 0.0};
+    if constexpr (!FULL) {
+        const int left = (int)a.R - (sub * NV * kWave + l) * 4;  // elements from this lane's first one on
+        const float kf = (float)Kd;
+#pragma unroll
+        for (int u = 0; u < NV; ++u)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) t[u][c] = u * kWave * 4 + c < left ? t[u][c] : kf;
+    }
 #pragma unroll
     for (int u = 0; u < NV; ++u) {
         const double d0 = (double)t[u].x - Kd, d1 = (double)t[u].y - Kd;
@@ -738,17 +767,31 @@ struct ColArgs {
 template <class Op, int VEC, int TX, int U, int BLK>
 __global__ __launch_bounds__(BLK) void k_cols(ColArgs a) {
     using Acc = typename Op::Acc;
+    using Final = typename Finish<Op>::Final;
     using State = typename Op::State;
     constexpr int TY = BLK / TX;
-    const float prm = a.fin.p;  // op parameter (NORM exponent)
+    float prm[VEC];  // op parameter (NORM exponent; var / std: the column's shift, its first row)
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) prm[j] = a.fin.p;
     const int tid = threadIdx.x;
     const int tx = tid % TX;
     const int ty = tid / TX;
     const int s = blockIdx.x % a.S;
     const long long ob = blockIdx.x / a.S;
-    const long long cb = ob % a.ncb;
-    const long long o = ob / a.ncb;
-    const long long col0 = (cb * TX + tx) * VEC;
+    long long cb = ob % a.ncb;
+    long long o = ob / a.ncb;
+    // The column blocks of one outer index on one XCD (unsplit workgroups go round
+    // the eight of them): where rows are not whole cache lines neighbouring blocks
+    // share a line at their edge, and its second reader finds it in that L2.
+    if (a.S == 1 && a.ncb > 1 && (o / 8 + 1) * 8 <= a.outer) {
+        const int w = (int)(ob - o / 8 * 8 * a.ncb);
+        o = o / 8 * 8 + w % 8;
+        cb = w / 8;
+    }
+    // the last vector of columns moves back inside the row; the columns it shares
+    // with its neighbour get the same result from both
+    const bool live = (cb * TX + tx) * VEC < a.inner;
+    const long long col0 = VEC == 1 ? cb * TX + tx : min((cb * TX + tx) * VEC, a.inner - VEC);
 
     Acc acc[VEC];
 #pragma unroll
@@ -757,41 +800,35 @@ __global__ __launch_bounds__(BLK) void k_cols(ColArgs a) {
     // rows of the reduced dim are interleaved over the TY thread rows and the S
     // splits (row r goes to split (r / TY) % S), so concurrently running
     // workgroups read neighbouring rows; U rows are in flight per thread
-    if (col0 < a.inner) {
+    if (live) {
         const float* base = a.in + o * a.os + col0;
         const int R = (int)a.R;
         const int rstep = TY * a.S;
-        const int r0 = s * TY + ty;
-        if (VEC == 4 && col0 + 3 < a.inner) {
-            int r = r0;
-            for (; r + (U - 1) * rstep < R; r += U * rstep) {
-                float4 t[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) t[u] = ld4(reinterpret_cast<const float4*>(base + (long long)(r + u * rstep) * a.rs), a.nt);
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int ru = r + u * rstep;
-                    Op::acc(acc[0], t[u].x, ru, prm);
-                    Op::acc(acc[1 % VEC], t[u].y, ru, prm);
-                    Op::acc(acc[2 % VEC], t[u].z, ru, prm);
-                    Op::acc(acc[3 % VEC], t[u].w, ru, prm);
-                }
+        auto ld = [&](float (&t)[VEC], int r) {
+            const float* q = base + (long long)r * a.rs;
+            if constexpr (VEC == 4) {
+                const float4 v = ld4(q, a.nt);
+                t[0] = v.x; t[1] = v.y; t[2] = v.z; t[3] = v.w;
+            } else {
+                t[0] = *q;
             }
-            for (; r < R; r += rstep) {
-                float4 t = *reinterpret_cast<const float4*>(base + (long long)r * a.rs);
-                Op::acc(acc[0], t.x, r, prm);
-                Op::acc(acc[1 % VEC], t.y, r, prm);
-                Op::acc(acc[2 % VEC], t.z, r, prm);
-                Op::acc(acc[3 % VEC], t.w, r, prm);
-            }
-        } else {
-            const int nj = (int)min((long long)VEC, a.inner - col0);
-            for (int r = r0; r < R; r += rstep) {
-                const float* q = base + (long long)r * a.rs;
+        };
+        if constexpr (Finish<Op>::kShift) ld(prm, 0);
+        int r = s * TY + ty;
+        for (; r + (U - 1) * rstep < R; r += U * rstep) {
+            float t[U][VEC];
 #pragma unroll
-                for (int j = 0; j < VEC; ++j)
-                    if (j < nj) Op::acc(acc[j], q[j], r, prm);
-            }
+            for (int u = 0; u < U; ++u) ld(t[u], r + u * rstep);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) Op::acc(acc[j], t[u][j], r + u * rstep, prm[j]);
+        }
+        for (; r < R; r += rstep) {
+            float t[VEC];
+            ld(t, r);
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) Op::acc(acc[j], t[j], r, prm[j]);
         }
     }
 
@@ -816,16 +853,14 @@ __global__ __launch_bounds__(BLK) void k_cols(ColArgs a) {
             __syncthreads();
         }
     }
-    if (ty == 0) {
+    if (ty == 0 && live) {
         const long long nout = a.outer * a.inner;
 #pragma unroll
         for (int j = 0; j < VEC; ++j) {
-            const long long c = col0 + j;
-            if (c < a.inner) {
-                const long long oi = o * a.inner + c;
-                if (!a.partial) fin_write(st[j], a.fin, a.out, oi);
-                else reinterpret_cast<State*>(a.part)[(long long)s * nout + oi] = shift_index(st[j], a.idx_off, 0);
-            }
+            const long long oi = o * a.inner + col0 + j;
+            const typename Final::State f = Finish<Op>::of(st[j], prm[j]);
+            if (!a.partial) fin_write(f, a.fin, a.out, oi);
+            else reinterpret_cast<typename Final::State*>(a.part)[(long long)s * nout + oi] = shift_index(f, a.idx_off, 0);
         }
     }
 }
@@ -915,6 +950,34 @@ struct AnyVec {
     typedef T type __attribute__((ext_vector_type(NV), aligned(sizeof(T))));
 };
 
+// Adds the NV elements of a vector, the first of index i.  Sums of 1-byte
+// integers add four bytes per instruction (v_dot4 against ones, 32 bits) and one
+// 64-bit value per vector: exact, and a 64-bit add per byte was what bounded
+// them ([8192, 8192] int8 row sums 15.8 -> 12.3 us).
+template <class Op, class T>
+struct ByteSum {
+    static constexpr bool value = false;
+};
+
+template <class Op, class T, int NV, class Vec>
+__device__ __forceinline__ void acc_vec(typename Op::Acc& acc, const Vec& t, int i, float prm) {
+    if constexpr (ByteSum<Op, T>::value) {
+        static_assert(NV == 16, "16 bytes");
+        int w[4];
+        __builtin_memcpy(w, &t, 16);
+        int c = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if constexpr (std::is_signed<T>::value) c = __builtin_amdgcn_sdot4(w[k], 0x01010101, c, false);
+            else c = (int)__builtin_amdgcn_udot4((unsigned)w[k], 0x01010101u, (unsigned)c, false);
+        }
+        acc += c;
+    } else {
+#pragma unroll
+        for (int k = 0; k < NV; ++k) Op::acc(acc, (T)t[k], i + k, prm);
+    }
+}
+
 template <class Op, class T, int NV, int BLK>
 __global__ __launch_bounds__(BLK) void k_runs(RunArgs a) {
     using Acc = typename Op::Acc;
@@ -967,10 +1030,7 @@ __global__ __launch_bounds__(BLK) void k_runs(RunArgs a) {
                 const unsigned q = u + k * ngrp;
                 if (q < a.units) {
                     const int j = (int)q * a.L;
-                    if (l < nv) {
-#pragma unroll
-                        for (int i = 0; i < NV; ++i) Op::acc(acc, (T)x[k][i], j + l * NV + i, prm);
-                    }
+                    if (l < nv) acc_vec<Op, T, NV>(acc, x[k], j + l * NV, prm);
                     if (nv * NV + l < a.L) Op::acc(acc, t[k], j + te, prm);
                 }
             }
@@ -991,10 +1051,7 @@ __global__ __launch_bounds__(BLK) void k_runs(RunArgs a) {
                 for (int k = 0; k < U; ++k) x[k] = *reinterpret_cast<const V*>(p + (long long)min(v + k * G, nv - 1) * NV);
 #pragma unroll
                 for (int k = 0; k < U; ++k) {
-                    if (v + k * G < nv) {
-#pragma unroll
-                        for (int i = 0; i < NV; ++i) Op::acc(acc, (T)x[k][i], j + (v + k * G) * NV + i, prm);
-                    }
+                    if (v + k * G < nv) acc_vec<Op, T, NV>(acc, x[k], j + (v + k * G) * NV, prm);
                 }
             }
             if (nv * NV + l < len) Op::acc(acc, t, j + te, prm);
@@ -1030,7 +1087,15 @@ __global__ __launch_bounds__(kBlock) void k_finalize_thread(FinArgs a) {
     if (o >= a.nout) return;
     const State* p = reinterpret_cast<const State*>(a.part);
     State st = p[o];
-    for (int s = 1; s < a.S; ++s) st = Op::comb(st, p[(long long)s * a.nout + o]);
+    int s = 1;
+    for (; s + 7 < a.S; s += 8) {  // eight loads in flight
+        State t[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) t[k] = p[(long long)(s + k) * a.nout + o];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) st = Op::comb(st, t[k]);
+    }
+    for (; s < a.S; ++s) st = Op::comb(st, p[(long long)s * a.nout + o]);
     fin_write(st, a.fin, a.out, o);
 }
 
@@ -1057,6 +1122,7 @@ struct Plan {
     int tx = 64;     // cols
     int unroll = 4;  // rows/cols: vectors in flight per thread
     int nt = 0;      // rows/cols: nontemporal input loads
+    bool rows16 = true;  // rows/cols: every row starts on a multiple of four elements from the first
     int colblock = 256;  // cols: threads per workgroup
     int reg_wpr = 0;     // rows: > 0 selects k_rows_reg with this many waves per row
     int var_nv = 0;      // rows, VAR/STD: > 0 selects k_rows_reg_var (float4 per lane; reg_wpr waves per row)
@@ -1233,7 +1299,7 @@ void plan_runs(Plan& p, int NV) {
     p.units = Q * p.nch;
 }
 
-Plan make_plan(const tpr_reduce_desc* d, const void* in) {
+Plan make_plan(const tpr_reduce_desc* d) {
     Plan p;
     p.state_bytes = state_size(d->op, d->p);
     const int nd = d->ndim;
@@ -1280,29 +1346,26 @@ Plan make_plan(const tpr_reduce_desc* d, const void* in) {
     const bool ordered = d->op == TPR_ARGMAX || d->op == TPR_ARGMIN ||
                          ((d->op == TPR_AMAX || d->op == TPR_AMIN || d->op == TPR_NORM) &&
                           (d->in_dtype == TPR_FLOAT32 || d->in_dtype == TPR_FLOAT64));
-    if (!ordered)
-        std::stable_sort(Rd.d, Rd.d + Rd.n,
-                         [](const Dim& x, const Dim& y) { return std::llabs(x.stride) > std::llabs(y.stride); });
+    if (!ordered) {
+        for (int i = 1; i < Rd.n; ++i)
+            for (int j = i; j > 0 && std::llabs(Rd[j].stride) > std::llabs(Rd[j - 1].stride); --j) std::swap(Rd[j], Rd[j - 1]);
+    }
     // Kept (and reduced) dims that continue each other merge across whatever
     // lay between them: outputs are row-major over the kept dims, and reduced
     // indices over the reduced dims.
     auto merge = [](Dims& v) {
-        Dims m;
-        for (auto& x : v) {
-            if (!m.empty() && m.back().stride == x.stride * x.size) {
-                m.back().size *= x.size;
-                m.back().stride = x.stride;
-            } else {
-                m.push_back(x);
-            }
+        int n = 0;
+        for (int i = 1; i < v.n; ++i) {
+            const Dim x = v[i];
+            if (v[n].stride == x.stride * x.size) v[n] = Dim{v[n].size * x.size, x.stride, x.red};
+            else v[++n] = x;
         }
-        v = m;
+        if (v.n > 0) v.n = n + 1;
     };
     merge(K);
     merge(Rd);
 
     const auto& dev = device_info();
-    const bool aligned16 = (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
     const bool force_general = knobs().general != 0;
     const bool empty = (p.count == 0 || p.nout == 0);
 
@@ -1344,7 +1407,8 @@ Plan make_plan(const tpr_reduce_desc* d, const void* in) {
         p.rows = K.empty() ? 1 : K[0].size;
         p.row_stride = K.empty() ? 0 : K[0].stride;
         p.R = Rd.empty() ? 1 : Rd[0].size;
-        p.vec = (aligned16 && (p.rows == 1 || p.row_stride % 4 == 0) && p.R >= 4) ? 4 : 1;
+        p.vec = 4;  // rows start and end at any element
+        p.rows16 = p.rows == 1 || p.row_stride % 4 == 0;
         // lanes per row: >= ~32 elements per thread, and enough lanes that the
         // grid holds ~4096 threads per CU; rows are split over workgroups only
         // when even 256 lanes per row leave fewer than ~512 threads per CU
@@ -1366,7 +1430,7 @@ Plan make_plan(const tpr_reduce_desc* d, const void* in) {
         // 32 lanes with exactly 8 vectors each (rows of 1024 floats): all eight
         // in flight at once (C2 var / std / argmax dim=-1 on MI355X: 41.7 /
         // 41.8 / 40.6 us against 42.2 / 42.2 / 41.3 us with two tiles of 4)
-        if (lanes == 32 && p.vec == 4 && ceil_div(p.R, 4 * 32) == 8) p.unroll = 8;
+        if (lanes == 32 && ceil_div(p.R, 4 * 32) == 8) p.unroll = 8;
         const long long tiles = std::max(1LL, ceil_div(p.R, 16 * lanes));  // 4 vectors x 4 floats per lane
         long long threads = p.rows * lanes;
         long long S = 1;
@@ -1376,10 +1440,10 @@ Plan make_plan(const tpr_reduce_desc* d, const void* in) {
         // Zero-identity ops over rows of 65-1024 float4, with enough rows to give
         // every CU at least 8 waves: one burst of two 128-bit loads per lane,
         // WPR waves per row (k_rows_reg).  The workspace stays zero, as for S == 1.
-        const long long nv4 = p.R / 4;
+        const long long nv4 = ceil_div(p.R, 4);
         const bool zero_id = d->op == TPR_SUM || d->op == TPR_MEAN || d->op == TPR_ANY ||
                              (d->op == TPR_NORM && (d->p == 1.0 || d->p == 2.0));
-        if (zero_id && p.vec == 4 && p.R % 4 == 0 && nv4 > kWave && nv4 <= 1024 && knobs().rowreg >= 0 &&
+        if (zero_id && nv4 > kWave && nv4 <= 1024 && knobs().rowreg >= 0 &&
             knobs().splits <= 0 && knobs().lanes <= 0) {
             const long long wpr = std::max(1LL, pow2_ceil(ceil_div(nv4, 2 * kWave)));
             if (knobs().rowreg > 0 || p.rows * wpr >= (long long)dev.cus * 8) {
@@ -1387,15 +1451,16 @@ Plan make_plan(const tpr_reduce_desc* d, const void* in) {
                 p.S = 1;
             }
         }
-        // var / std over rows of 1024, 2048 or 4096 floats (1, 2 or 4 waves of
-        // four float4 per lane, exactly): the shifted two-sum kernel.  Measured
-        // on MI355X: C2 var dim=-1 [65536, 1024] 39.9 us against 42.6 us,
-        // [4096, 4096] 12.0 against 16.7 us, [16384, 2048] 21.6 against 23.3 us;
-        // two float4 per lane (rows of 512) was slower than k_rows (48 us).
-        if ((d->op == TPR_VAR || d->op == TPR_STD) && p.vec == 4 && p.R % 4 == 0 && nv4 % (4 * kWave) == 0 &&
+        // var / std over rows that fill three quarters or more of 1, 2 or 4 waves of
+        // four float4 per lane (769..1024, 1537..2048, 3073..4096 floats): the
+        // shifted two-sum kernel.  Measured on MI355X against WelfordOp in k_rows:
+        // C2 var dim=-1 [65536, 1024] 39.9 us against 42.6 us, [4096, 4096] 12.0
+        // against 16.7 us, [16384, 2048] 21.6 against 23.3 us; two float4 per lane
+        // (rows of 512) was slower than k_rows (48 us).
+        if ((d->op == TPR_VAR || d->op == TPR_STD) && d->in_dtype == TPR_FLOAT32 && p.R <= 16 * kWave * 4 &&
             knobs().rowreg >= 0 && knobs().splits <= 0 && knobs().lanes <= 0) {
-            const long long wv = nv4 / (4 * kWave);
-            if ((wv == 1 || wv == 2 || wv == 4) && (knobs().rowreg > 0 || p.rows * wv >= (long long)dev.cus * 8)) {
+            const long long wv = pow2_ceil(ceil_div(p.R, 16 * kWave));
+            if (4 * p.R > 3 * 16 * kWave * wv && (knobs().rowreg > 0 || p.rows * wv >= (long long)dev.cus * 8)) {
                 p.reg_wpr = (int)wv;
                 p.var_nv = 4;
                 p.S = 1;
@@ -1409,9 +1474,8 @@ Plan make_plan(const tpr_reduce_desc* d, const void* in) {
         p.os = (K.size() == 2) ? K[0].stride : 0;
         p.R = Rd[0].size;
         p.rs = Rd[0].stride;
-        p.vec = (aligned16 && p.rs % 4 == 0 && (p.outer == 1 || p.os % 4 == 0) && p.inner >= 4) ? 4 : 1;
-        // plan on float4 columns whatever the alignment, so the workspace size
-        // does not depend on the pointer
+        p.vec = p.inner >= 4 ? 4 : 1;  // rows start and end at any element
+        p.rows16 = p.rs % 4 == 0 && (p.outer == 1 || p.os % 4 == 0);
         const long long cols4 = ceil_div(p.inner, 4);
         const long long target = (long long)dev.cus * 512;
         if (p.outer * ceil_div(cols4, 256) * kBlock >= target || p.R < 16) p.tx = 256;
@@ -1483,7 +1547,9 @@ int launch_rows_reg_var(const Plan& p, const float* in, void* out, Fin fin, hipS
     const int wpr = p.reg_wpr;
 #define TPR_VAR_CASE(NV, WPR, BLK)                                                                             \
     if (nv == NV && wpr == WPR) {                                                                              \
-        hipLaunchKernelGGL((k_rows_reg_var<NV, WPR, BLK>), dim3(ceil_div(p.rows, BLK / (kWave * WPR))), dim3(BLK), 0, st, a); \
+        const dim3 g(ceil_div(p.rows, BLK / (kWave * WPR)));                                                    \
+        if (p.R == 4 * kWave * NV * WPR) hipLaunchKernelGGL((k_rows_reg_var<NV, WPR, BLK, true>), g, dim3(BLK), 0, st, a); \
+        else hipLaunchKernelGGL((k_rows_reg_var<NV, WPR, BLK, false>), g, dim3(BLK), 0, st, a);                 \
         return check_launch("k_rows_reg_var");                                                                 \
     }
     TPR_VAR_CASE(4, 1, 256) TPR_VAR_CASE(4, 2, 256) TPR_VAR_CASE(4, 4, 256)
@@ -1494,7 +1560,7 @@ int launch_rows_reg_var(const Plan& p, const float* in, void* out, Fin fin, hipS
 template <class Op>
 int launch_rows(const Plan& p, const float* in, void* out, void* ws, Fin fin, hipStream_t st,
                 unsigned* tickets = nullptr) {
-    if constexpr (std::is_same<Op, WelfordOp>::value) {
+    if constexpr (std::is_same<Op, WelfordOp>::value || std::is_same<Op, ShiftVarOp>::value) {
         if (p.var_nv > 0) return launch_rows_reg_var(p, in, out, fin, st);
     }
     if constexpr (kZeroIdentity<Op>) {
@@ -1509,11 +1575,10 @@ int launch_rows(const Plan& p, const float* in, void* out, void* ws, Fin fin, hi
 #define TPR_ROWS_CASE(L)                                                                             \
     case L: {                                                                                        \
         constexpr int B = L > kBlock ? L : kBlock;                                                   \
-        if (L == 32 && p.vec == 4 && p.unroll == 8) hipLaunchKernelGGL((k_rows<Op, 4, (L == 32 ? 32 : 16), 8>), dim3(grid), dim3(B), 0, st, a); \
-        else if (p.vec == 4 && p.unroll == 1) hipLaunchKernelGGL((k_rows<Op, 4, L, 1>), dim3(grid), dim3(B), 0, st, a); \
-        else if (p.vec == 4 && p.unroll == 2) hipLaunchKernelGGL((k_rows<Op, 4, L, 2>), dim3(grid), dim3(B), 0, st, a); \
-        else if (p.vec == 4) hipLaunchKernelGGL((k_rows<Op, 4, L, 4>), dim3(grid), dim3(B), 0, st, a); \
-        else hipLaunchKernelGGL((k_rows<Op, 1, L, 4>), dim3(grid), dim3(B), 0, st, a);             \
+        if (L == 32 && p.unroll == 8) hipLaunchKernelGGL((k_rows<Op, (L == 32 ? 32 : 16), 8>), dim3(grid), dim3(B), 0, st, a); \
+        else if (p.unroll == 1) hipLaunchKernelGGL((k_rows<Op, L, 1>), dim3(grid), dim3(B), 0, st, a); \
+        else if (p.unroll == 2) hipLaunchKernelGGL((k_rows<Op, L, 2>), dim3(grid), dim3(B), 0, st, a); \
+        else hipLaunchKernelGGL((k_rows<Op, L, 4>), dim3(grid), dim3(B), 0, st, a);                \
         break;                                                                                       \
     }
     switch (p.lanes) {
@@ -1657,6 +1722,15 @@ unsigned* fused_split_tickets(const Plan& p, hipStream_t st) {
 }
 
 template <class Op>
+int launch_layout(const Plan& p, const float* in, void* out, void* ws, Fin fin, hipStream_t st, unsigned* tk) {
+    switch (p.kind) {
+        case P_ROWS: return launch_rows<Op>(p, in, out, ws, fin, st, tk);
+        case P_COLS: return launch_cols<Op>(p, in, out, ws, fin, st);
+        default: return launch_runs<Op, float, 4>(p, in, out, ws, fin, st, tk);
+    }
+}
+
+template <class Op>
 int run(const Plan& p, const float* in, void* out, void* ws, Fin fin, hipStream_t st) {
     if (p.nchunk > 1)
         return run_chunks<Op>(p, in, sizeof(float), out, ws, fin, st, [&](const Plan& pc, const void* ic, void* wc) {
@@ -1665,17 +1739,11 @@ int run(const Plan& p, const float* in, void* out, void* ws, Fin fin, hipStream_
         });
     int rc = TPR_OK;
     unsigned* tk = fused_split_tickets(p, st);
-    if (p.kind == P_ROWS) rc = launch_rows<Op>(p, in, out, ws, fin, st, tk);
-    else if (p.kind == P_COLS) rc = launch_cols<Op>(p, in, out, ws, fin, st);
-    else if (p.kind == P_RUNS) {
-        if constexpr (std::is_same<Op, WelfordOp>::value) {
-            rc = p.count <= kShiftMax ? launch_runs<ShiftVarOp, float, 4>(p, in, out, ws, fin, st, tk)
-                                      : launch_runs<Op, float, 4>(p, in, out, ws, fin, st, tk);
-        } else {
-            rc = launch_runs<Op, float, 4>(p, in, out, ws, fin, st, tk);
-        }
-    }
-    else rc = launch_general<Op>(p, in, out, ws, fin, st);
+    if (p.kind == P_GENERAL) rc = launch_general<Op>(p, in, out, ws, fin, st);
+    else if (std::is_same<Op, WelfordOp>::value && p.count <= kShiftMax)
+        rc = launch_layout<typename std::conditional<std::is_same<Op, WelfordOp>::value, ShiftVarOp, Op>::type>(
+            p, in, out, ws, fin, st, tk);
+    else rc = launch_layout<Op>(p, in, out, ws, fin, st, tk);
     if (rc != TPR_OK) return rc;
     if (p.S > 1 && !tk) rc = launch_finalize<Op>(p, out, ws, fin, st);
     return rc;
@@ -1715,6 +1783,11 @@ struct IntSumOp {
     __device__ static State identity() { return {PROD ? 1 : 0}; }
     __device__ static State comb(State a, State b) { return {PROD ? wrap_mul(a.s, b.s) : wrap_add(a.s, b.s)}; }
     __device__ static State shfl(State s, int m) { return {lane_xor(s.s, m)}; }
+};
+
+template <class T>
+struct ByteSum<IntSumOp<T, false>, T> {
+    static constexpr bool value = sizeof(T) == 1;
 };
 
 // Mean of an integer input: the reference converts the input to Float32 first
@@ -1836,25 +1909,22 @@ struct ArgsI {
     unsigned* tickets;  // as RowArgs (rows only)
 };
 
-template <class T, int NV>
-struct alignas(16) Vec16 {
-    T v[NV];
-};
-
-// 16-byte nontemporal load of NV elements (the row kernel's read-once
-// stream).  Measured on MI355X: float64 full reductions of 2^27 elements 171 ->
-// 155 us against plain loads; the column kernel keeps plain loads (nontemporal
-// ones were 2-6% slower there: int32 sum over dim 1 of [64, 1024, 1024] 44.9
-// against 42.4 us).  A runtime choice between the two is not possible here: the
-// compiler merges the two otherwise identical loads of the branches into one
-// and drops the nontemporal mark.
-template <class T, int NV>
-__device__ __forceinline__ Vec16<T, NV> ld16_nt(const Vec16<T, NV>* p) {
+// 16-byte loads of NV elements, starting at any element.  NT: nontemporal (the
+// row kernel's read-once stream).  Measured on MI355X: float64 full reductions
+// of 2^27 elements 171 -> 155 us against plain loads; the column kernel keeps
+// plain loads (nontemporal ones were 2-6% slower there: int32 sum over dim 1 of
+// [64, 1024, 1024] 44.9 against 42.4 us).  A template parameter: the compiler
+// merges the two otherwise identical loads of a runtime choice into one and
+// drops the nontemporal mark.
+template <bool NT, class T, int NV>
+__device__ __forceinline__ void ld16(T (&t)[NV], const T* p) {
+    using V = typename AnyVec<T, NV>::type;
+    V r;
+    if constexpr (NT) r = __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
+    else r = *reinterpret_cast<const V*>(p);
     typedef int i32x4 __attribute__((ext_vector_type(4)));
-    Vec16<T, NV> t;
-    const i32x4 r = __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(p));
-    __builtin_memcpy(&t, &r, 16);
-    return t;
+    const i32x4 w = __builtin_bit_cast(i32x4, r);
+    __builtin_memcpy(&t, &w, 16);
 }
 
 template <class Op, int LANES>
@@ -1881,7 +1951,7 @@ __device__ __forceinline__ typename Op::State combine_lanes(typename Op::State s
 }
 
 // Row kernel for integer inputs: [rows, R], R contiguous; NV elements per
-// 16-byte vector (1 = scalar loads).  Split s takes vectors s*LANES + l + k*S*LANES.
+// 16-byte vector, rows starting and ending at any element.  Split s takes vectors s*LANES + l + k*S*LANES.
 template <class Op, class T, int NV, int LANES>
 __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void k_rows_i(ArgsI a) {
     using Acc = typename Op::Acc;
@@ -1898,31 +1968,24 @@ __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void k_rows_i(Args
     if (row < a.rows) {
         const T* p = static_cast<const T*>(a.in) + row * a.row_stride;
         const int R = (int)a.R;
-        int tail = 0;
-        if constexpr (NV > 1) {
-            const int nv = R / NV;
-            const Vec16<T, NV>* pv = reinterpret_cast<const Vec16<T, NV>*>(p);
-            const int step = a.S * LANES;
-            int v = s * LANES + l;
-            // four vectors in flight per lane; each lane still visits its
-            // elements in increasing index order
-            for (; v + 3 * step < nv; v += 4 * step) {
-                Vec16<T, NV> t[4];
+        const int nv = R / NV;
+        const int step = a.S * LANES;
+        int v = s * LANES + l;
+        // four vectors in flight per lane; each lane still visits its
+        // elements in increasing index order
+        for (; v + 3 * step < nv; v += 4 * step) {
+            T t[4][NV];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) t[u] = ld16_nt(pv + v + u * step);
+            for (int u = 0; u < 4; ++u) ld16<true>(t[u], p + (long long)(v + u * step) * NV);
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-#pragma unroll
-                    for (int j = 0; j < NV; ++j) Op::acc(acc, t[u].v[j], (v + u * step) * NV + j, prm);
-            }
-            for (; v < nv; v += step) {
-                const Vec16<T, NV> t = ld16_nt(pv + v);
-#pragma unroll
-                for (int j = 0; j < NV; ++j) Op::acc(acc, t.v[j], v * NV + j, prm);
-            }
-            tail = nv * NV;
+            for (int u = 0; u < 4; ++u) acc_vec<Op, T, NV>(acc, t[u], (v + u * step) * NV, prm);
         }
-        for (int e = tail + s * LANES + l; e < R; e += a.S * LANES) Op::acc(acc, p[e], e, prm);
+        for (; v < nv; v += step) {
+            T t[NV];
+            ld16<true>(t, p + (long long)v * NV);
+            acc_vec<Op, T, NV>(acc, t, v * NV, prm);
+        }
+        for (int e = nv * NV + s * LANES + l; e < R; e += a.S * LANES) Op::acc(acc, p[e], e, prm);
     }
     using State = typename Op::State;
     State st = combine_lanes<Op, LANES>(Op::state(acc), tid);
@@ -1954,40 +2017,37 @@ __global__ __launch_bounds__(kBlock) void k_cols_i(ArgsI a) {
     const long long ob = blockIdx.x / a.S;
     const long long cb = ob % a.ncb;
     const long long o = ob / a.ncb;
-    const long long col0 = (cb * TX + tx) * NV;
+    // the last vector of columns moves back inside the row, as in k_cols
+    const bool live = (cb * TX + tx) * NV < a.inner;
+    const long long col0 = NV == 1 ? cb * TX + tx : min((cb * TX + tx) * NV, a.inner - NV);
     Acc acc[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j) acc[j] = Op::init();
-    if (col0 < a.inner) {
+    if (live) {
         const T* base = static_cast<const T*>(a.in) + o * a.os + col0;
         const int R = (int)a.R;
         const int rstep = TY * a.S;
-        if (NV > 1 && col0 + NV <= a.inner) {
-            int r = s * TY + ty;
-            // four rows in flight per thread, visited in increasing row order
-            for (; r + 3 * rstep < R; r += 4 * rstep) {
-                Vec16<T, NV> t[4];
+        auto ld = [&](T (&t)[NV], int r) {
+            const T* q = base + (long long)r * a.rs;
+            if constexpr (NV > 1) ld16<false>(t, q);
+            else t[0] = *q;
+        };
+        int r = s * TY + ty;
+        // four rows in flight per thread, visited in increasing row order
+        for (; r + 3 * rstep < R; r += 4 * rstep) {
+            T t[4][NV];
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    t[u] = *reinterpret_cast<const Vec16<T, NV>*>(base + (long long)(r + u * rstep) * a.rs);
+            for (int u = 0; u < 4; ++u) ld(t[u], r + u * rstep);
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < 4; ++u)
 #pragma unroll
-                    for (int j = 0; j < NV; ++j) Op::acc(acc[j], t[u].v[j], r + u * rstep, prm);
-            }
-            for (; r < R; r += rstep) {
-                const Vec16<T, NV> t = *reinterpret_cast<const Vec16<T, NV>*>(base + (long long)r * a.rs);
+                for (int j = 0; j < NV; ++j) Op::acc(acc[j], t[u][j], r + u * rstep, prm);
+        }
+        for (; r < R; r += rstep) {
+            T t[NV];
+            ld(t, r);
 #pragma unroll
-                for (int j = 0; j < NV; ++j) Op::acc(acc[j], t.v[j], r, prm);
-            }
-        } else {
-            const int nj = (int)min((long long)NV, a.inner - col0);
-            for (int r = s * TY + ty; r < R; r += rstep) {
-                const T* q = base + (long long)r * a.rs;
-#pragma unroll
-                for (int j = 0; j < NV; ++j)
-                    if (j < nj) Op::acc(acc[j], q[j], r, prm);
-            }
+            for (int j = 0; j < NV; ++j) Op::acc(acc[j], t[j], r, prm);
         }
     }
     State st[NV];
@@ -2009,16 +2069,13 @@ __global__ __launch_bounds__(kBlock) void k_cols_i(ArgsI a) {
             __syncthreads();
         }
     }
-    if (ty == 0) {
+    if (ty == 0 && live) {
         const long long nout = a.outer * a.inner;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-            const long long c = col0 + j;
-            if (c < a.inner) {
-                const long long oi = o * a.inner + c;
-                if (!a.partial) fin_write(st[j], a.fin, a.out, oi);
-                else reinterpret_cast<State*>(a.part)[(long long)s * nout + oi] = shift_index(st[j], a.idx_off, 0);
-            }
+            const long long oi = o * a.inner + col0 + j;
+            if (!a.partial) fin_write(st[j], a.fin, a.out, oi);
+            else reinterpret_cast<State*>(a.part)[(long long)s * nout + oi] = shift_index(st[j], a.idx_off, 0);
         }
     }
 }
@@ -2206,16 +2263,15 @@ size_t int_state_size(int op) {
 // vector).  Rows: lanes rounded up to 16/64/256/1024.  Columns: 256-thread
 // workgroups, TX 64/128/256, splits recomputed on NV-wide columns.  The
 // workspace size depends on the descriptor only, never on the pointer.
-void adapt_plan_int(Plan& p, const tpr_reduce_desc* d, const void* in, int es) {
+void adapt_plan_int(Plan& p, const tpr_reduce_desc* d, int es) {
     const int NV = 16 / es;
-    const bool aligned16 = (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
     const auto& dev = device_info();
     const long long target = (long long)dev.cus * 512;
     p.state_bytes = d->in_dtype == TPR_FLOAT64 ? f64_state_size(d->op, d->p) : int_state_size(d->op);
     p.reg_wpr = 0;  // the register-row kernels read float32 only
     p.var_nv = 0;
     if (p.kind == P_ROWS) {
-        p.vec = (aligned16 && (p.rows == 1 || p.row_stride % NV == 0) && p.R >= NV) ? NV : 1;
+        p.vec = NV;
         int L = 16;
         while (L < p.lanes && L < 1024) L *= 4;
         p.lanes = L;
@@ -2225,7 +2281,7 @@ void adapt_plan_int(Plan& p, const tpr_reduce_desc* d, const void* in, int es) {
             p.S = threads < target ? std::max(1LL, std::min(ceil_div(target, threads), vecs)) : 1;
         }
     } else if (p.kind == P_COLS) {
-        p.vec = (aligned16 && p.rs % NV == 0 && (p.outer == 1 || p.os % NV == 0) && p.inner >= NV) ? NV : 1;
+        p.vec = p.inner >= NV ? NV : 1;
         p.colblock = kBlock;
         const long long colsv = ceil_div(p.inner, NV);
         if (!(knobs().tx == 64 || knobs().tx == 128 || knobs().tx == 256))
@@ -2258,8 +2314,7 @@ int launch_int_layout(const Plan& p, const void* in, void* out, void* ws, Fin fi
         const dim3 blk(p.lanes > kBlock ? p.lanes : kBlock);
 #define TPR_ROWS_I(L)                                                                               \
     case L:                                                                                         \
-        if (p.vec > 1) hipLaunchKernelGGL((k_rows_i<Op, T, NV, L>), grid, blk, 0, st, a);          \
-        else hipLaunchKernelGGL((k_rows_i<Op, T, 1, L>), grid, blk, 0, st, a);                     \
+        hipLaunchKernelGGL((k_rows_i<Op, T, NV, L>), grid, blk, 0, st, a);                         \
         break;
         switch (p.lanes) {
             TPR_ROWS_I(16)
@@ -2694,10 +2749,9 @@ extern "C" {
 
 size_t tpr_reduce_workspace_bytes(const tpr_reduce_desc* desc) {
     if (tpr::validate(desc) != TPR_OK) return 0;
-    // alignment does not change the workspace size; plan with an aligned pointer
-    tpr::Plan p = tpr::make_plan(desc, nullptr);
+    tpr::Plan p = tpr::make_plan(desc);
     if (desc->op == TPR_MEDIAN) return p.count > 0 ? tpr::median_ws_bytes(p.count, nullptr) : 0;
-    if (desc->in_dtype != TPR_FLOAT32) tpr::adapt_plan_int(p, desc, nullptr, tpr::esize_of(desc->in_dtype));
+    if (desc->in_dtype != TPR_FLOAT32) tpr::adapt_plan_int(p, desc, tpr::esize_of(desc->in_dtype));
     return p.ws;
 }
 
@@ -2706,14 +2760,18 @@ int tpr_reduce(const tpr_reduce_desc* desc, const void* in, void* out, void* wor
     using namespace tpr;
     int rc = validate(desc);
     if (rc != TPR_OK) return rc;
-    Plan p = make_plan(desc, in);
+    Plan p = make_plan(desc);
     if (p.nout == 0) return TPR_OK;
     if (!out) return fail(TPR_ERR_INVALID_ARG, "tpr_reduce: null output");
     if (!in && p.count > 0) return fail(TPR_ERR_INVALID_ARG, "tpr_reduce: null input");
+    // Vectors off 16 bytes share cache lines with their neighbours, which a
+    // nontemporal line may not wait for ([63, 1021, 1023], five reductions: 236 us
+    // nontemporal, 209 plain).
+    if (knobs().nt == 0 && ((reinterpret_cast<uintptr_t>(in) & 15) != 0 || !p.rows16)) p.nt = 0;
     if (desc->op == TPR_MEDIAN)
         return run_median(desc, p, in, out, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
     const bool int_in = desc->in_dtype != TPR_FLOAT32;
-    if (int_in) adapt_plan_int(p, desc, in, esize_of(desc->in_dtype));
+    if (int_in) adapt_plan_int(p, desc, esize_of(desc->in_dtype));
     if (p.ws > 0 && (workspace == nullptr || workspace_bytes < p.ws))
         return fail(TPR_ERR_WORKSPACE, "tpr_reduce: workspace too small (need " +
                                            std::to_string(p.ws) + " bytes)");

@@ -1,0 +1,67 @@
+"""Row and column reductions whose rows start and end at any element: the vector
+loads at unaligned addresses, the row's tail, the last column vector moved back
+inside the row, and var / std shifted by one element, against the general
+kernel (as test_reduce_runs_gpu.py) and float64."""
+import numpy as np
+import pytest
+
+from tensorplay_amd import _capi
+from tests.test_reduce_runs_gpu import _no_knob, both  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def view(shape, off, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    buf = torch.randn((shape[0], shape[1] + off + 3), generator=g) * 20
+    buf = buf.round() if dtype != torch.float32 else buf
+    return buf.to(dtype).cuda()[:, off:off + shape[1]]
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 6, 7, 63, 65, 130, 257, 1022, 1023, 1025, 4099, 20001])
+@pytest.mark.parametrize("off", [0, 1, 2])
+def test_float_rows_and_columns(n, off):
+    rows = 3 if n > 4000 else 70
+    x = view((rows, n), off, torch.float32, n)
+    for op in ("sum", "amax", "argmin", "var", "norm", "any"):
+        both(x, op, [1])
+        both(x, op, [0])
+    both(x.contiguous(), "argmax", None)
+    both(x.contiguous(), "std", None)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.int64, torch.int32, torch.int16, torch.int8, torch.uint8])
+@pytest.mark.parametrize("n", [1, 3, 15, 17, 33, 127, 1023, 4097])
+def test_other_types(dtype, n):
+    x = view((41, n), 1, dtype, n).abs() if dtype == torch.uint8 else view((41, n), 1, dtype, n)
+    for op in ("sum", "amax", "argmax"):
+        both(x, op, [1])
+        both(x, op, [0])
+
+
+@pytest.mark.parametrize("rows", [2000, 70000])
+def test_register_rows_of_odd_length(rows):
+    for n in (261, 1023, 2047):
+        if rows * n > 40_000_000:
+            continue
+        x = view((rows, n), 3, torch.float32, n)
+        for op in ("sum", "mean", "any"):
+            both(x, op, [1])
+
+
+@pytest.mark.parametrize("shape,dims", [((300, 1023), [1]), ((1023, 300), [0]), ((40, 77, 129), [0, 2]), ((9, 5000), [1])])
+def test_shifted_variance_error(shape, dims):
+    """Against float64: a mean far above the spread, and a first element (the
+    shift) that is the set's outlier.  The shifted sums lose at most about n 2^-53
+    of M2, far below the float32 result's rounding (2^-24)."""
+    g = torch.Generator().manual_seed(4)
+    for mean, outlier in ((0.0, 0.0), (1e4, 0.0), (0.0, 1e6)):
+        x = torch.randn(shape, generator=g) + mean
+        first = [0 if d in dims else slice(None) for d in range(x.dim())]
+        x[tuple(first)] += outlier
+        ref = x.double().var(dims).numpy()
+        got = _capi.reduce(x.cuda(), "var", dims).cpu().numpy()
+        np.testing.assert_allclose(got, ref, rtol=2.0 ** -23)
+        got = _capi.reduce(x.cuda(), "std", dims).cpu().numpy()
+        np.testing.assert_allclose(got, np.sqrt(ref), rtol=2.0 ** -22)
