@@ -33,9 +33,11 @@
 //   * longer rows stream twice: an online (max, sum-of-exp) pass, then the
 //     output pass -- k_smx_rows2, or split over (row, chunk) workgroups when
 //     the rows are fewer than the CUs -- k_smx_part / k_smx_apply;
-//   * strided forward slices of 513..1024 rows with 16-byte columns: two row
+//   * strided forward slices of 513..1024 rows: two row
 //     pieces per 64-column group exchanging per-column statistics --
 //     k_smx_cols4p;
+//   * strided gradients of 257..1024 rows: pieces of 256 rows exchanging
+//     per-column sums -- k_smx_cols4pb;
 //   * a strided softmax dim (inner extent > 1, or a non-unit dim stride)
 //     keeps one column per lane, thread rows across the dim, an LDS merge of
 //     the per-wave states, and also streams twice -- k_smx_cols.
@@ -651,6 +653,7 @@ __global__ __launch_bounds__(kResT) void k_smx_res_bwd(SmxArgs p, int vl) {
 // ---------------------------------------------------------------------------
 constexpr int kPcMax = 16;                     // most pieces per row
 constexpr int kFwdPcVR = 20;                   // forward pieces: float4 of x per lane
+constexpr int kColPcMax = 4;                   // most pieces per strided slice
 constexpr int kSmxSlots = 1 << 18;             // exchange slots (2 MiB); a launch never needs more
 
 }  // namespace
@@ -1124,8 +1127,9 @@ __global__ __launch_bounds__(kWave * BY) void k_smx_cols(SmxColArgs p) {
     }
 }
 
-// Strided dim with a contiguous, 16-byte aligned inner dim (inner % 4 == 0):
-// a wave covers 4 rows x 64 columns (16 lanes of float4 per row, 256 bytes
+// Strided dim with a contiguous inner dim of at least 16 columns, rows at any
+// float (the last float4 of a row moves back inside it, and writes the same
+// values as its neighbour): a wave covers 4 rows x 64 columns (16 lanes of float4 per row, 256 bytes
 // contiguous), BY waves split the dim, 64 columns per workgroup.  Per-thread
 // online states per float4 component, merged across the wave's 4 row lanes by
 // shuffles and across waves through LDS in a fixed order.
@@ -1140,9 +1144,10 @@ __global__ __launch_bounds__(kWave * BY) void k_smx_cols4(SmxColArgs p) {
     const int w = threadIdx.x / kWave;
     const int cl = lane % 16, rl = lane / 16;
     const long long ncg = (p.inner + 63) / 64;
-    const long long o = blockIdx.x / ncg;
-    const long long c = (blockIdx.x - o * ncg) * 64 + 4 * cl;  // first column of this lane
+    const long long o = blockIdx.x / (unsigned)ncg;  // the grid is outer * ncg < 2^31
+    long long c = (blockIdx.x - o * ncg) * 64 + 4 * cl;  // first column of this lane
     const bool live = c < p.inner;
+    if (live) c = min(c, p.inner - 4);  // the last vector moves back inside the row: shared columns, equal values
     const float* pa = p.a + o * p.a_so + (live ? c : 0);
     const float* pb = BW ? p.b + o * p.b_so + (live ? c : 0) : nullptr;
     float* po = p.out + o * p.n * p.inner + (live ? c : 0);
@@ -1253,9 +1258,10 @@ __global__ __launch_bounds__(kWave * BY) void k_smx_cols4r(SmxColArgs p) {
     const int w = threadIdx.x / kWave;
     const int cl = lane % CW, rl = lane / CW;
     const long long ncg = (p.inner + 4 * CW - 1) / (4 * CW);
-    const long long o = blockIdx.x / ncg;
-    const long long c = (blockIdx.x - o * ncg) * (4 * CW) + 4 * cl;  // first column of this lane
+    const long long o = blockIdx.x / (unsigned)ncg;  // the grid is outer * ncg < 2^31
+    long long c = (blockIdx.x - o * ncg) * (4 * CW) + 4 * cl;  // first column of this lane
     const bool live = c < p.inner;
+    if (live) c = min(c, p.inner - 4);  // the last vector moves back inside the row: shared columns, equal values
     const float* pa = p.a + o * p.a_so + (live ? c : 0);
     const float* pb = BW ? p.b + o * p.b_so + (live ? c : 0) : nullptr;
     float* po = p.out + o * p.n * p.inner + (live ? c : 0);
@@ -1469,9 +1475,10 @@ __global__ __launch_bounds__(kWave * BY) __attribute__((amdgpu_waves_per_eu(4, 8
     const long long ncg = (p.inner + 4 * CW - 1) / (4 * CW);
     const long long gi = blockIdx.x / 2;  // column group
     const int pc = (int)(blockIdx.x % 2);
-    const long long o = gi / ncg;
-    const long long c = (gi - o * ncg) * (4 * CW) + 4 * cl;
+    const long long o = (unsigned)gi / (unsigned)ncg;
+    long long c = (gi - o * ncg) * (4 * CW) + 4 * cl;
     const bool live = c < p.inner;
+    if (live) c = min(c, p.inner - 4);  // the last vector moves back inside the row: shared columns, equal values
     const float* pa = p.a + o * p.a_so + (live ? c : 0);
     float* po = p.out + o * p.n * p.inner + (live ? c : 0);
     const int n = live ? (int)p.n : 0;
@@ -1571,6 +1578,127 @@ __global__ __launch_bounds__(kWave * BY) __attribute__((amdgpu_waves_per_eu(4, 8
             const float xv[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
 #pragma unroll
             for (int q = 0; q < 4; ++q) out[q] = outv<MODE>(xv[q], 0.0f, st0[q], st1[q]);
+            vst<4, NT>(po + (long long)r * p.inner, out);
+        }
+    }
+}
+
+// Gradients along a strided dim of 257..1024 rows: as k_smx_cols4p, each 64-column
+// group is cut into np pieces of RS * V rows, one workgroup each holding its g and
+// y in registers (V = 8: 64 of them for the data, two workgroups per CU), so both
+// cross HBM once where k_smx_cols4 reads them twice.  Only a sum per column (g . y,
+// or g) is exchanged.  MI355X, [64, 1024, 1024] dim 1: 216 -> 156 us.
+template <int MODE, int BY, int V, bool NT>
+__global__ __launch_bounds__(kWave * BY) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_smx_cols4pb(SmxColArgs p, int np, unsigned epoch, int spin) {
+    static_assert(MODE == BWD || MODE == BWD_LOG, "gradients only");
+    constexpr int CW = 16, RW = kWave / CW, RS = RW * BY, PR = RS * V;  // PR rows per piece
+    __shared__ f32x4 shs[BY][CW];
+    __shared__ f32x4 ps[kColPcMax][CW];
+    __shared__ unsigned missing;
+    const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave, cl = lane % CW, rl = lane / CW;
+    const long long ncg = (p.inner + 4 * CW - 1) / (4 * CW);
+    const long long gi = blockIdx.x / np;  // column group
+    const int pc = (int)(blockIdx.x % np);
+    const long long o = (unsigned)gi / (unsigned)ncg;
+    long long c = (gi - o * ncg) * (4 * CW) + 4 * cl;
+    const bool live = c < p.inner;
+    if (live) c = min(c, p.inner - 4);
+    const float* pa = p.a + o * p.a_so + (live ? c : 0);
+    const float* pb = p.b + o * p.b_so + (live ? c : 0);
+    float* po = p.out + o * p.n * p.inner + (live ? c : 0);
+    const int n = live ? (int)p.n : 0;
+    auto row_of = [&](int piece, int i) { return piece * PR + rl + RW * w + i * RS; };
+    auto term = [](const float (&x)[4], const float (&z)[4], f32x4& acc) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] += MODE == BWD ? x[q] * z[q] : x[q];
+    };
+    // a piece's column sums: lanes, then waves in order (valid in every thread)
+    auto merge = [&](f32x4 acc) {
+#pragma unroll
+        for (int off = CW; off <= 32; off <<= 1)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc[q] += xor_lane_f(acc[q], off);
+        __syncthreads();  // shs may still be read from an earlier call
+        if (rl == 0) shs[w][cl] = acc;
+        __syncthreads();
+        f32x4 t = shs[0][cl];
+        for (int k = 1; k < BY; ++k) t += shs[k][cl];
+        return t;
+    };
+    float g[V][4], y[V][4];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int r = row_of(pc, i);
+        if (r < n) {
+            vld<4, NT>(g[i], pa + (long long)r * p.a_sn);
+            vld<4, NT>(y[i], pb + (long long)r * p.b_sn);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) g[i][q] = y[i][q] = 0.0f;
+        }
+    }
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < V; ++i) term(g[i], y[i], acc);
+    const f32x4 own = merge(acc);
+    if (w == 0 && rl == 0) {
+        ps[pc][cl] = own;
+        unsigned long long* slot = smx_slots;
+        const long long base = gi * np * CW * 4 + cl * 4;  // + piece * CW * 4 + q
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            __hip_atomic_exchange(slot + ((base + pc * CW * 4 + q) & (kSmxSlots - 1)),
+                                  ((unsigned long long)epoch << 32) | __float_as_uint(own[q]), __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+        unsigned need = ((1u << (4 * np)) - 1u) & ~(0xfu << (4 * pc));  // bit 4 * piece + q: not seen yet
+        const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+        for (;;) {
+            for (int j = 0; j < 4 * np; ++j) {
+                if (!((need >> j) & 1u)) continue;
+                const unsigned long long v = __hip_atomic_fetch_or(
+                    slot + ((base + (j >> 2) * CW * 4 + (j & 3)) & (kSmxSlots - 1)), 0ull, __ATOMIC_RELAXED,
+                    __HIP_MEMORY_SCOPE_AGENT);
+                if ((unsigned)(v >> 32) == epoch) {
+                    reinterpret_cast<float*>(&ps[j >> 2][cl])[j & 3] = __uint_as_float((unsigned)v);
+                    need &= ~(1u << j);
+                }
+            }
+            if (need == 0 || __builtin_amdgcn_s_memrealtime() - t0 > (unsigned long long)spin) break;
+            __builtin_amdgcn_s_sleep(2);
+        }
+        // any of the 16 owner lanes short of a piece: the whole workgroup recomputes it
+        unsigned short_of = 0;
+        for (int k = 0; k < np; ++k) short_of |= __ballot(((need >> (4 * k)) & 0xfu) != 0) != 0ull ? 1u << k : 0u;
+        if (lane == 0) missing = short_of;
+    }
+    __syncthreads();
+    const unsigned miss = missing;
+    for (int k = 0; k < np; ++k) {
+        if (!((miss >> k) & 1u)) continue;  // uniform
+        f32x4 a2 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma nounroll
+        for (int i = 0; i < V; ++i) {
+            const int r = row_of(k, i);
+            float x[4] = {0.0f, 0.0f, 0.0f, 0.0f}, z[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (r < n) {
+                vld<4, false>(x, pa + (long long)r * p.a_sn);
+                vld<4, false>(z, pb + (long long)r * p.b_sn);
+            }
+            term(x, z, a2);
+        }
+        a2 = merge(a2);
+        if (w == 0 && rl == 0) ps[k][cl] = a2;
+        __syncthreads();
+    }
+    f32x4 dot = ps[0][cl];
+    for (int k = 1; k < np; ++k) dot += ps[k][cl];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int r = row_of(pc, i);
+        if (r < n) {
+            float out[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) out[q] = outv<MODE>(g[i][q], y[i][q], dot[q], 0.0f);
             vst<4, NT>(po + (long long)r * p.inner, out);
         }
     }
@@ -1897,6 +2025,9 @@ template <int MODE>
 int run_rows(const SmxArgs& a0, int vw, hipStream_t st) {
     SmxArgs a = a0;
     const int two_pass = knobs().smx_two_pass;
+    // rows off 16 bytes whose output lies over an input keep the kernels that
+    // never read a row again after another workgroup may have written it
+    const bool pieces_ok = vw == 4 || (a.out != a.a && a.out != a.b);
     // gradients: g and y both held (row pieces over workgroups), each read once
     if constexpr (MODE >= BWD) {
         // 512-thread pieces of 24 float4 per lane; measured on MI355X (us):
@@ -1906,7 +2037,7 @@ int run_rows(const SmxArgs& a0, int vw, hipStream_t st) {
         // (one slot per piece: a launch whose pieces outnumber the slots would
         // reuse a slot under the same epoch, so it takes the kernels below)
         const int ns = row_pieces(a.n, 512, 24, st);
-        if (ns > 0 && a.rows * ns <= kSmxSlots) return launch_bwd_pieces<MODE, 512, 24>(a, ns, st);
+        if (ns > 0 && pieces_ok && a.rows * ns <= kSmxSlots) return launch_bwd_pieces<MODE, 512, 24>(a, ns, st);
     } else if (knobs().smx_fwd_pieces >= 0) {
         // forward: x held by row pieces when the one-row-per-CU kernel below
         // would take more than one round and a row makes two pieces or more;
@@ -1924,7 +2055,7 @@ int run_rows(const SmxArgs& a0, int vw, hipStream_t st) {
         // -> 237, log 230 -> 150 and 309 -> 225).  The test
         // knob smx_fwd_pieces = 1 takes every row the pieces can hold.
         const int ns = row_pieces(a.n, 512, kFwdPcVR, st);
-        if (ns > 0 && a.rows * ns * 2 <= kSmxSlots &&  // two slots per piece, none reused in a launch
+        if (ns > 0 && pieces_ok && a.rows * ns * 2 <= kSmxSlots &&  // two slots per piece, none reused in a launch
             (knobs().smx_fwd_pieces > 0 || vw != 4 || (ns >= 2 && a.rows > device_info().cus) ||
              (a.n > kResMax && knobs().smx_fwd_pieces == 0)))
             return launch_fwd_pieces<MODE, 512, kFwdPcVR>(a, ns, st);
@@ -1967,12 +2098,18 @@ int run_rows(const SmxArgs& a0, int vw, hipStream_t st) {
 }
 
 template <int MODE>
-int run_cols(const SmxColArgs& a, hipStream_t st) {
+int run_cols(const SmxColArgs& a_in, hipStream_t st) {
     constexpr bool BW = MODE >= BWD;
+    SmxColArgs a = a_in;
     auto al = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-    const bool v4 = a.a_si == 1 && a.inner % 4 == 0 && a.inner >= 16 && al(a.a) && al(a.out) && a.a_so % 4 == 0 &&
-                    a.a_sn % 4 == 0 && (!BW || (a.b_si == 1 && al(a.b) && a.b_so % 4 == 0 && a.b_sn % 4 == 0)) &&
-                    knobs().general == 0;
+    const bool al16 = a.inner % 4 == 0 && al(a.a) && al(a.out) && a.a_so % 4 == 0 && a.a_sn % 4 == 0 &&
+                      (!BW || (al(a.b) && a.b_so % 4 == 0 && a.b_sn % 4 == 0));
+    // an output over one of its inputs keeps the kernels in which a column has one
+    // reader and writer, where vectors would share columns
+    const bool alias = a.out == a.a || a.out == a.b;
+    const bool v4 = a.a_si == 1 && (!BW || a.b_si == 1) && a.inner >= 16 && (al16 || !alias) && knobs().general == 0;
+    // vectors off 16 bytes share cache lines, which a nontemporal line may not wait for
+    if (!al16 && knobs().nt == 0) a.nt = 0;
     if (v4) {
         const long long blocks = a.outer * ((a.inner + 63) / 64);
         if (blocks <= 0x7fffffffLL) {
@@ -1994,7 +2131,36 @@ int run_cols(const SmxColArgs& a, hipStream_t st) {
                     return check_launch("tpr_softmax (strided dim, row pieces)");
                 }
             }
-            if (a.n > 64 && a.n <= (BW ? 256 : 1024) && knobs().smx_res >= 0 && knobs().smx_two_pass == 0) {
+            if constexpr (BW) {
+                // gradients of slices of 257..1024 rows: pieces of 256 rows, launched
+                // over as many outer indices at a time as have slots of their own
+                const long long ncg = (a.inner + 63) / 64;
+                const int np = (int)((a.n + 255) / 256);
+                const long long per = kSmxSlots / (ncg * np * 64);
+                if (a.n > 256 && np <= kColPcMax && knobs().smx_res >= 0 && knobs().smx_two_pass == 0 &&
+                    knobs().smx_pieces >= 0 && per > 0 && !alias && !capturing(st)) {
+                    const int spin = knobs().smx_spin < 0 ? 0 : 4000;
+                    for (long long o0 = 0; o0 < a.outer; o0 += per) {
+                        SmxColArgs b = a;
+                        b.outer = std::min(per, a.outer - o0);
+                        b.a += o0 * a.a_so;
+                        b.b += o0 * a.b_so;
+                        b.out += o0 * a.n * a.inner;
+                        unsigned ep = smx_epoch_ctr.fetch_add(1, std::memory_order_relaxed) + 1u;
+                        if (ep == 0) ep = smx_epoch_ctr.fetch_add(1, std::memory_order_relaxed) + 1u;
+                        const dim3 g((unsigned)(b.outer * ncg * np)), blk(kWave * 8);
+                        if (a.nt) hipLaunchKernelGGL((k_smx_cols4pb<MODE, 8, 8, true>), g, blk, 0, st, b, np, ep, spin);
+                        else hipLaunchKernelGGL((k_smx_cols4pb<MODE, 8, 8, false>), g, blk, 0, st, b, np, ep, spin);
+                        const int rc = check_launch("tpr_softmax (strided dim gradient, row pieces)");
+                        if (rc != TPR_OK) return rc;
+                    }
+                    return TPR_OK;
+                }
+            }
+            if (a.n <= (BW ? 256 : 1024) && knobs().smx_res >= 0 && knobs().smx_two_pass == 0) {
+                // up to 64 rows: as few waves as hold them, four rows per lane (two
+                // passes of k_smx_cols4, 4 waves, before: [16, 21, 512, 512] dim 1 270 -> 133
+                // us, gradient 220 -> 193; [16, 8, 256, 256] 51 -> 15.5)
                 // 64-column groups (CW = 16); 32-column groups (CW = 8, two
                 // workgroups per CU) measured slower: 143 vs 131 us at [64, 1024,
                 // 1024] dim 1, 193 vs 111 us at [2048, 128, 256]
@@ -2004,7 +2170,10 @@ int run_cols(const SmxColArgs& a, hipStream_t st) {
         if (a.nt) hipLaunchKernelGGL((k_smx_cols4r<MODE, BYV, VV, 16, true>), dim3(g), dim3(kWave * BYV), 0, st, a); \
         else hipLaunchKernelGGL((k_smx_cols4r<MODE, BYV, VV, 16, false>), dim3(g), dim3(kWave * BYV), 0, st, a); \
     }
-                if (a.n <= 128) TPR_C4R(8, 4)
+                if (a.n <= 16) TPR_C4R(1, 4)
+                else if (a.n <= 32) TPR_C4R(2, 4)
+                else if (a.n <= 64) TPR_C4R(4, 4)
+                else if (a.n <= 128) TPR_C4R(8, 4)
                 else if (a.n <= 256) TPR_C4R(8, 8)
                 else if constexpr (!BW) {
                     if (a.n <= 512) TPR_C4R(16, 8)
