@@ -46,6 +46,9 @@ constexpr int kBlock = 256;
 // of kTicketsPerStream counters for each of up to kTicketStreams streams.
 constexpr int kTicketStreams = 64;
 constexpr int kTicketsPerStream = 1024;
+constexpr int kTicketGroups = 16;
+constexpr int kTicketSpread = 32;  // counters of 128 bytes
+static_assert((kTicketGroups + 1) * kTicketSpread <= kTicketsPerStream, "a stream's block holds the group counters");
 
 // ---------------------------------------------------------------------------
 // Operator policies.  Acc = per-thread running state, State = mergeable state.
@@ -349,6 +352,11 @@ __device__ __forceinline__ typename Op::State block_reduce_n(typename Op::State 
 // performed at the device's point of coherence, so no L2 writeback or
 // invalidate is needed (such fences cost microseconds per workgroup), and the
 // wait for the exchanges to complete (vmcnt(0)) orders them before the ticket.
+// Tickets drawn from one word follow each other at about 9 ns, 4.6 us for the 512
+// workgroups of a full reduction that end together: a single output's splits
+// draw from one of kTicketGroups counters, each on its own 128 bytes, and the
+// last of each group from the output's.  MI355X, full sum of 2.4 M floats
+// 9.7 -> 5.2 us, of 16.8 M 16.6 -> 13.0, of 16.8 M bytes 10.9 -> 6.2.
 // ---------------------------------------------------------------------------
 template <class State>
 __device__ __forceinline__ void publish_state(State* dst, const State& v) {
@@ -384,7 +392,20 @@ __device__ void split_finish(typename Op::State st, typename Op::State* part, un
     if (tid == 0) {
         publish_state(part + (long long)s * stride + o, st);
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
+        auto draw = [](unsigned* t) {
+            return __hip_atomic_fetch_add(t, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        if (stride == 1 && S >= 4 * kTicketGroups) {
+            const int g = s % kTicketGroups;
+            unsigned* t = ticket + (g + 1) * kTicketSpread;
+            last = 0;
+            if (draw(t) == (unsigned)((S - g + kTicketGroups - 1) / kTicketGroups - 1)) {
+                __hip_atomic_store(t, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                last = draw(ticket) == (unsigned)(kTicketGroups - 1);
+            }
+        } else {
+            last = draw(ticket) == (unsigned)(S - 1);
+        }
     }
     __syncthreads();
     if (!last) return;
