@@ -32,7 +32,7 @@
 // instructions an element) and the fixed tail (sort, scans).  512 threads, so
 // that a thread may hold 216 of a row's values (54 float4, 252 registers).
 // MI355X, k = cols, against the sort of all candidates in the workspace that
-// this replaced: [256, 151936] T 0.8 top_p 0.9 6070 -> 86 us, [256, 50257] 1075
+// this replaced: [256, 151936] T 0.8 top_p 0.9 6070 -> 80 us, [256, 50257] 1075
 // -> 42, [1, 151936] 3976 -> 50; the radix draws (T 1, top_p 1) 275 / 92 / 153.
 #include <hip/hip_runtime.h>
 
@@ -49,6 +49,7 @@ namespace {
 constexpr int kNT = 512;      // threads per row
 constexpr int kNW = kNT / 64;
 constexpr int kList = 4096;   // candidates sorted in phase 3 (8 per thread)
+constexpr int kListK = 1600;  // largest k tried on a list cut by the bound of phase 2
 constexpr int kBins = 2048;
 
 typedef float f4 __attribute__((ext_vector_type(4)));
@@ -327,7 +328,8 @@ __device__ void draw_by_radix(SampleShared& sh, const float* p, int n, float v0,
 }
 
 // m and the draw from the sorted list; false if the list does not reach the
-// nucleus end.
+// nucleus end.  A negative total: the list holds the top k, whose weight is the
+// list's own.
 __device__ bool draw_from_list(SampleShared& sh, int cnt, int k, float v0, double total, float u, const SampleArgs& a,
                                long long* out) {
     constexpr int P = kList / kNT;
@@ -359,6 +361,12 @@ __device__ bool draw_from_list(SampleShared& sh, int cnt, int k, float v0, doubl
     for (int i = 0; i < kNW; ++i)
         if (i < w) before += sh.dsum[i];
     const double excl = before + (incl - s);
+    const bool whole = total < 0.0;
+    if (whole) {
+        total = 0.0;
+#pragma unroll
+        for (int i = 0; i < kNW; ++i) total += sh.dsum[i];
+    }
     const double cut = (double)a.top_p * total;
     int mj = 0x7fffffff;
     double c = excl;
@@ -367,8 +375,11 @@ __device__ bool draw_from_list(SampleShared& sh, int cnt, int k, float v0, doubl
         c += pw[q];
         if (c >= cut && mj == 0x7fffffff && t * P + q <= last) mj = t * P + q;
     }
-    const int m = block_min(mj, sh.wmin[0]);
-    if (m > last) return false;
+    int m = block_min(mj, sh.wmin[0]);
+    if (m > last) {
+        if (!whole) return false;
+        m = last;  // c_{k-1} reaches the cut whatever the roundings
+    }
     c = excl;
 #pragma unroll
     for (int q = 0; q < P; ++q) {
@@ -453,6 +464,29 @@ __global__ __launch_bounds__(kNT) void k_sample_row(SampleArgs a) {
     uint32_t kth = 0;  // every element is above key 0
     u64 kties = 0;
     if constexpr (!ALL) {
+        // Small k: the bound that keeps the list short (phase 2) often leaves the
+        // whole top k on it -- about 1700 elements reach it -- and the sorted list
+        // then is the answer, where the k-th key costs three more passes
+        // ([64, 16000] k = 1050 48 -> 36 us, [64, 151936] 141 ->
+        // 101).  Rows of kList or less would sort all of themselves ([64, 2097]
+        // 33 against 25).
+        if (n > kList && a.k <= kListK) {
+            stream_row(p, 0, n, [&](float v, int i) {
+                if (v >= lo) {
+                    const int at = atomicAdd(&sh.count, 1);
+                    if (at < kList) sh.list[at] = comp_key(f2key(v, 1), (uint32_t)i);
+                }
+            });
+            __syncthreads();
+            const int cnt = sh.count;
+            __syncthreads();
+            if (cnt >= a.k && cnt <= kList) {
+                draw_from_list(sh, cnt, a.k, v0, -1.0, u, a, &a.ids[row]);
+                return;
+            }
+            if (t == 0) sh.count = 0;
+            __syncthreads();
+        }
         const Pick r = pick_rank(sh, p, n, (u64)a.k, a);
         kth = r.key;
         kties = (u64)a.k - r.above;
@@ -483,14 +517,35 @@ __global__ __launch_bounds__(kNT) void k_sample_row(SampleArgs a) {
         u64 hits = 0;
 #pragma unroll
         for (int j = 0; j < VR; ++j) hits |= add(x[j]) ? 1ull << j : 0ull;
-        while (hits) {  // few: read again rather than indexed in the registers
-            const int i = 4 * ((__ffsll(hits) - 1) * kNT + t);
-            hits &= hits - 1;
-            const f4 v = *reinterpret_cast<const f4u*>(p + i);
-            for (int c = 0; c < 4; ++c) list(v[c], i + c);
+        // few: read again, four at a time, rather than indexed in the registers
+        while (hits) {
+            int i[4];
+            f4 v[4];
+            const int first = __ffsll(hits) - 1;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int j = hits ? __ffsll(hits) - 1 : -1;
+                hits &= hits - 1;
+                i[q] = j < 0 ? -1 : 4 * (j * kNT + t);
+                v[q] = *reinterpret_cast<const f4u*>(p + 4 * ((j < 0 ? first : j) * kNT + t));
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (i[q] >= 0)
+                    for (int c = 0; c < 4; ++c) list(v[q][c], i[q] + c);
         }
         const int nv = n >> 2;
-        for (int i = VR * kNT + t; i < nv; i += kNT) {
+        int i = VR * kNT + t;
+        for (; i + 7 * kNT < nv; i += 8 * kNT) {  // eight vectors in flight
+            f4 v[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = *reinterpret_cast<const f4u*>(p + 4ll * (i + q * kNT));
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                if (add(v[q]))
+                    for (int c = 0; c < 4; ++c) list(v[q][c], 4 * (i + q * kNT) + c);
+        }
+        for (; i < nv; i += kNT) {
             const f4 v = *reinterpret_cast<const f4u*>(p + 4ll * i);
             if (add(v))
                 for (int c = 0; c < 4; ++c) list(v[c], 4 * i + c);

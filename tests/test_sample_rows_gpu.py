@@ -20,7 +20,8 @@ def logits(rng, rows, cols, scale=2.0):
     return x
 
 
-@pytest.mark.parametrize("cols", [1025, 2047, 6 * V - 1, 6 * V, 14 * V + 1, 24 * V, 36 * V + 3, 54 * V, 54 * V + 4 * V + 2])
+@pytest.mark.parametrize("cols", [1025, 2047, 6 * V - 1, 6 * V, 14 * V + 1, 24 * V, 36 * V + 3, 54 * V, 54 * V + 4 * V + 2,
+                                  62 * V - 1, 62 * V, 62 * V + 5, 71 * V + 3])
 @pytest.mark.parametrize("T,top_p", [(0.8, 0.9), (1.0, 1.0), (0.0, 0.5)])
 def test_row_lengths(cols, T, top_p):
     rng = np.random.default_rng(cols)
