@@ -216,7 +216,7 @@ __global__ __launch_bounds__(kNllBlock) void k_nll_bwd_rows(NllBwdArgs a) {
 
 // Shorter rows (n * c < 2^32 - 1024): one 32-bit division per vector.  [8192,
 // 1000]: one element per thread with a 64-bit division each took 12.7 us, this
-// this 6.7 us.
+// 6.7 us.
 __global__ __launch_bounds__(kNllBlock) void k_nll_bwd_short(NllBwdArgs a) {
     const unsigned e = (blockIdx.x * (unsigned)kNllBlock + threadIdx.x) * 4u;
     const unsigned c = (unsigned)a.c, total = (unsigned)(a.n * a.c);
