@@ -1237,6 +1237,7 @@ __global__ __launch_bounds__(kBlock) void k_finalize_block(FinArgs a) {
 // ---------------------------------------------------------------------------
 // Host planner.
 // ---------------------------------------------------------------------------
+constexpr long long kColsVecMin = 4 << 20;  // bytes (cols_vec)
 enum PlanKind { P_ROWS = 1, P_COLS = 2, P_GENERAL = 3, P_RUNS = 4, P_FEW_COLS = 5 };
 
 struct Plan {
@@ -1436,6 +1437,17 @@ void plan_runs(Plan& p, int NV) {
     p.units = Q * p.nch;
 }
 
+// Columns per thread of the column kernels: a 16-byte vector at any element.
+// Below 4 MiB a launch has too few columns to fill the chip that way; rows off 16
+// bytes then take one column per thread (MI355X, us, vectors / one column: int8
+// [197, 19, 57] argmax over 0 12.7 / 7.1, float32 7.7 / 4.5, float32 [466, 38, 17]
+// argmax over 1 6.3 / 4.4; from 6 MB on vectors win or tie).
+int cols_vec(const Plan& p, int nv) {
+    if (p.inner < nv) return 1;
+    const bool rows16 = p.rs % nv == 0 && (p.outer == 1 || p.os % nv == 0);
+    return rows16 || p.count * p.nout * (16 / nv) > kColsVecMin ? nv : 1;
+}
+
 Plan make_plan(const tpr_reduce_desc* d) {
     Plan p;
     p.state_bytes = state_size(d->op, d->p);
@@ -1620,8 +1632,8 @@ Plan make_plan(const tpr_reduce_desc* d) {
         p.os = (K.size() == 2) ? K[0].stride : 0;
         p.R = Rd[0].size;
         p.rs = Rd[0].stride;
-        p.vec = p.inner >= 4 ? 4 : 1;  // rows start and end at any element
         p.rows16 = p.rs % 4 == 0 && (p.outer == 1 || p.os % 4 == 0);
+        p.vec = cols_vec(p, 4);
         const long long cols4 = ceil_div(p.inner, 4);
         const long long target = (long long)dev.cus * 512;
         if (p.outer * ceil_div(cols4, 256) * kBlock >= target || p.R < 16) p.tx = 256;
@@ -2439,7 +2451,7 @@ void adapt_plan_int(Plan& p, const tpr_reduce_desc* d, int es) {
             p.S = threads < target ? std::max(1LL, std::min(ceil_div(target, threads), vecs)) : 1;
         }
     } else if (p.kind == P_COLS) {
-        p.vec = p.inner >= NV ? NV : 1;
+        p.vec = cols_vec(p, NV);
         p.colblock = kBlock;
         const long long colsv = ceil_div(p.inner, NV);
         if (!(knobs().tx == 64 || knobs().tx == 128 || knobs().tx == 256))

@@ -65,3 +65,17 @@ def test_shifted_variance_error(shape, dims):
         np.testing.assert_allclose(got, ref, rtol=2.0 ** -23)
         got = _capi.reduce(x.cuda(), "std", dims).cpu().numpy()
         np.testing.assert_allclose(got, np.sqrt(ref), rtol=2.0 ** -22)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.int32, torch.int16, torch.int8])
+@pytest.mark.parametrize("inner", [129, 517])
+def test_columns_of_odd_rows_above_the_vector_bound(dtype, inner):
+    """More than 4 MiB: 16-byte column vectors where smaller calls take single columns."""
+    size = torch.empty(0, dtype=dtype).element_size()
+    rows = (5 << 20) // (size * inner * 131) + 1
+    x = view((rows * 131, inner), 1, dtype, inner)
+    for shape, dims in (((rows, 131, inner), (0, 1)), ((rows * 131, inner), (0,))):
+        y = x.as_strided(shape, ((131 * x.stride(0), x.stride(0), 1) if len(shape) == 3 else (x.stride(0), 1)), x.storage_offset())
+        for d in dims:
+            for op in ("sum", "amax", "argmax") + (("var",) if dtype in (torch.float32, torch.float64) else ()):
+                both(y, op, [d])
