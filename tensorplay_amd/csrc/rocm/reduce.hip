@@ -47,6 +47,7 @@ constexpr int kBlock = 256;
 constexpr int kTicketStreams = 64;
 constexpr int kTicketsPerStream = 1024;
 constexpr int kTicketGroups = 16;
+constexpr long long kGroupBytes = 256LL << 20;
 constexpr int kTicketSpread = 32;  // counters of 128 bytes
 static_assert((kTicketGroups + 1) * kTicketSpread <= kTicketsPerStream, "a stream's block holds the group counters");
 
@@ -355,7 +356,9 @@ __device__ __forceinline__ typename Op::State block_reduce_n(typename Op::State 
 // Tickets drawn from one word follow each other at about 9 ns, 4.6 us for the 512
 // workgroups of a full reduction that end together: a single output's splits
 // draw from one of kTicketGroups counters, each on its own 128 bytes, and the
-// last of each group from the output's.  MI355X, full sum of 2.4 M floats
+// last of each group from the output's.  Above kGroupBytes the workgroups end far
+// enough apart, and the second draw only adds its latency (six reductions of 1 GiB
+// 925.5 -> 930 us).  MI355X, full sum of 2.4 M floats
 // 9.7 -> 5.2 us, of 16.8 M 16.6 -> 13.0, of 16.8 M bytes 10.9 -> 6.2.
 // ---------------------------------------------------------------------------
 template <class State>
@@ -381,30 +384,37 @@ __device__ __forceinline__ State fetch_state(State* src) {
     return v;
 }
 
+// Output o's counter in a stream's block: neighbours on lines of their own.
+__device__ __forceinline__ unsigned* ticket_of(unsigned* tickets, long long o) {
+    constexpr int kLines = kTicketsPerStream / kTicketSpread;
+    return tickets + (o % kLines) * kTicketSpread + o / kLines;
+}
+
+__device__ __forceinline__ unsigned draw_ticket(unsigned* t) {
+    return __hip_atomic_fetch_add(t, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // st: the workgroup's partial state of output o (valid in thread 0); partial s
-// of output o lives at part[s * stride + o].
+// of output o lives at part[s * stride + o].  bytes: the input of one output.
 template <class Op, int BLK, class Fn>
 __device__ void split_finish(typename Op::State st, typename Op::State* part, unsigned* ticket, int S, int s,
-                             long long stride, long long o, Fn&& write) {
+                             long long stride, long long o, long long bytes, Fn&& write) {
     using State = typename Op::State;
     __shared__ int last;
     const int tid = threadIdx.x;
     if (tid == 0) {
         publish_state(part + (long long)s * stride + o, st);
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        auto draw = [](unsigned* t) {
-            return __hip_atomic_fetch_add(t, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        };
-        if (stride == 1 && S >= 4 * kTicketGroups) {
+        if (stride == 1 && S >= 4 * kTicketGroups && bytes <= kGroupBytes) {
             const int g = s % kTicketGroups;
             unsigned* t = ticket + (g + 1) * kTicketSpread;
             last = 0;
-            if (draw(t) == (unsigned)((S - g + kTicketGroups - 1) / kTicketGroups - 1)) {
+            if (draw_ticket(t) == (unsigned)((S - g + kTicketGroups - 1) / kTicketGroups - 1)) {
                 __hip_atomic_store(t, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                last = draw(ticket) == (unsigned)(kTicketGroups - 1);
+                last = draw_ticket(ticket) == (unsigned)(kTicketGroups - 1);
             }
         } else {
-            last = draw(ticket) == (unsigned)(S - 1);
+            last = draw_ticket(ticket) == (unsigned)(S - 1);
         }
     }
     __syncthreads();
@@ -589,8 +599,8 @@ __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void k_rows(RowArg
     const State st = Finish<Op>::of(os, prm);
     if constexpr (GROUPS == 1) {
         if (a.tickets) {
-            split_finish<Final, BLK>(st, reinterpret_cast<State*>(a.part), a.tickets + row, a.S, s, a.rows, row,
-                                  [&](const State& r) { fin_write(r, a.fin, a.out, row); });
+            split_finish<Final, BLK>(st, reinterpret_cast<State*>(a.part), ticket_of(a.tickets, row), a.S, s, a.rows, row,
+                                     a.R * (long long)sizeof(float), [&](const State& r) { fin_write(r, a.fin, a.out, row); });
             return;
         }
     }
@@ -1081,8 +1091,8 @@ __global__ __launch_bounds__(BLK) void k_runs(RunArgs a) {
     }
     const State st = Finish<Op>::of(block_reduce_n<Op, BLK>(Op::state(acc)), prm);
     if (a.tickets) {
-        split_finish<Final, BLK>(st, reinterpret_cast<State*>(a.part), a.tickets + o, a.S, s, a.nout, o,
-                              [&](const State& r) { fin_write(r, a.fin, a.out, o); });
+        split_finish<Final, BLK>(st, reinterpret_cast<State*>(a.part), ticket_of(a.tickets, o), a.S, s, a.nout, o, 0,
+                                 [&](const State& r) { fin_write(r, a.fin, a.out, o); });
         return;
     }
     if (threadIdx.x == 0) {
@@ -1102,8 +1112,8 @@ __global__ __launch_bounds__(BLK) void k_runs(RunArgs a) {
 // through LDS: entry e = NV * t + i has column e % inner, so every inner-th entry
 // belongs together; thread (c, m) adds entries m, m + M, ... of column c, then
 // the M slices meet in a tree.  Split s takes vectors s, s + S, ... of T threads.
-// MI355X, uint8 [64, 224, 224, 3] amax over 1, 2: 454 us -> 14, of which
-// k_few_cols 9.4 and k_finalize_thread 4.8.
+// MI355X, uint8 [64, 224, 224, 3] amax over 1, 2: 454 us -> 11.3 (9.4 and
+// 4.8 with k_finalize_thread after it).
 // ---------------------------------------------------------------------------
 struct FewColArgs {
     const void* in;
@@ -1112,6 +1122,7 @@ struct FewColArgs {
     void* out;
     void* part;
     Fin fin;
+    unsigned* tickets;  // S > 1: one counter per outer index (else null)
 };
 
 template <class Op, class T, int NV>
@@ -1183,14 +1194,41 @@ __global__ __launch_bounds__(kBlock) void k_few_cols(FewColArgs a) {
         __syncthreads();
         w = half;
     }
+    using FS = typename Final::State;
+    const long long oi = o * a.inner + t;
+    FS* part = reinterpret_cast<FS*>(a.part);
     if (t < a.inner) {
         float k = 0.0f;
         if constexpr (Finish<Op>::kShift) k = (float)p[t];
-        const typename Final::State f = Finish<Op>::of(sh[t], k);
-        const long long oi = o * a.inner + t;
+        const FS f = Finish<Op>::of(sh[t], k);
         if (a.S == 1) fin_write(f, a.fin, a.out, oi);
-        else reinterpret_cast<typename Final::State*>(a.part)[(long long)s * a.nout + oi] = f;
+        else if (a.tickets) publish_state(part + (long long)s * a.nout + oi, f);
+        else part[(long long)s * a.nout + oi] = f;
     }
+    if (a.S == 1 || !a.tickets) return;
+    // as split_finish, one thread per column; the columns combine their splits in
+    // order, as k_finalize_thread
+    __shared__ int last;
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    unsigned* ticket = ticket_of(a.tickets, o);
+    if (t == 0) last = draw_ticket(ticket) == (unsigned)(a.S - 1);
+    __syncthreads();
+    if (!last) return;
+    if (t < a.inner) {
+        FS r = fetch_state(part + oi);
+        int q = 1;
+        for (; q + 7 < a.S; q += 8) {
+            FS x[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) x[k] = fetch_state(part + (long long)(q + k) * a.nout + oi);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) r = Final::comb(r, x[k]);
+        }
+        for (; q < a.S; ++q) r = Final::comb(r, fetch_state(part + (long long)q * a.nout + oi));
+        fin_write(r, a.fin, a.out, oi);
+    }
+    if (t == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---------------------------------------------------------------------------
@@ -1832,8 +1870,8 @@ int launch_runs(const Plan& p, const void* in, void* out, void* ws, Fin fin, hip
 }
 
 template <class Op, class T, int NV>
-int launch_few_cols(const Plan& p, const void* in, void* out, void* ws, Fin fin, hipStream_t st) {
-    FewColArgs a{in, p.outer, p.os, p.nout, (int)p.R, (int)p.inner, p.lanes, (int)p.S, out, ws, fin};
+int launch_few_cols(const Plan& p, const void* in, void* out, void* ws, Fin fin, hipStream_t st, unsigned* tickets) {
+    FewColArgs a{in, p.outer, p.os, p.nout, (int)p.R, (int)p.inner, p.lanes, (int)p.S, out, ws, fin, tickets};
     hipLaunchKernelGGL((k_few_cols<Op, T, NV>), dim3(p.outer * p.S), dim3(kBlock), 0, st, a);
     return check_launch("k_few_cols");
 }
@@ -1875,11 +1913,13 @@ int run_chunks(const Plan& p, const void* in, size_t esize, void* out, void* ws,
 unsigned* stream_tickets(hipStream_t st);
 
 // Counters for a split plan that finishes in its own launch (split_finish):
-// row plans with S > 1 and one row per workgroup and run plans with S > 1, on a
+// row plans with S > 1 and one row per workgroup, run and few-column plans with S > 1, on a
 // stream that has a counter block.  Null: the plan takes the separate finalize
 // launch.
 unsigned* fused_split_tickets(const Plan& p, hipStream_t st) {
     if (p.S <= 1 || p.nchunk > 1 || p.partial) return nullptr;
+    // few columns: a thread combines a column's splits, so not many
+    if (p.kind == P_FEW_COLS) return p.outer <= kTicketsPerStream && p.S <= 64 ? stream_tickets(st) : nullptr;
     if (p.kind == P_RUNS) return p.nout <= kTicketsPerStream ? stream_tickets(st) : nullptr;
     if (p.kind != P_ROWS || p.lanes < kBlock || p.reg_wpr > 0 || p.var_nv > 0 || p.rows > kTicketsPerStream)
         return nullptr;
@@ -1891,7 +1931,7 @@ int launch_layout(const Plan& p, const float* in, void* out, void* ws, Fin fin, 
     switch (p.kind) {
         case P_ROWS: return launch_rows<Op>(p, in, out, ws, fin, st, tk);
         case P_COLS: return launch_cols<Op>(p, in, out, ws, fin, st);
-        case P_FEW_COLS: return launch_few_cols<Op, float, 4>(p, in, out, ws, fin, st);
+        case P_FEW_COLS: return launch_few_cols<Op, float, 4>(p, in, out, ws, fin, st, tk);
         default: return launch_runs<Op, float, 4>(p, in, out, ws, fin, st, tk);
     }
 }
@@ -2160,8 +2200,8 @@ __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void k_rows_i(Args
     State st = combine_lanes<Op, LANES>(Op::state(acc), tid);
     if constexpr (GROUPS == 1) {
         if (a.tickets) {
-            split_finish<Op, BLK>(st, reinterpret_cast<State*>(a.part), a.tickets + row, a.S, s, a.rows, row,
-                                  [&](const State& r) { fin_write(r, a.fin, a.out, row); });
+            split_finish<Op, BLK>(st, reinterpret_cast<State*>(a.part), ticket_of(a.tickets, row), a.S, s, a.rows, row,
+                                  a.R * (long long)sizeof(T), [&](const State& r) { fin_write(r, a.fin, a.out, row); });
             return;
         }
     }
@@ -2515,7 +2555,7 @@ int launch_int_layout(const Plan& p, const void* in, void* out, void* ws, Fin fi
     } else if (p.kind == P_RUNS) {
         return launch_runs<Op, T, NV>(p, in, out, ws, fin, st, tickets);
     } else if (p.kind == P_FEW_COLS) {
-        return launch_few_cols<Op, T, NV>(p, in, out, ws, fin, st);
+        return launch_few_cols<Op, T, NV>(p, in, out, ws, fin, st, tickets);
     } else {
         GenArgsI a{};
         a.in = in; a.nk = p.nk; a.nr = p.nr;
