@@ -27,9 +27,9 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, 8 TB/s
 # kernel each headline op launches (one launch per op: the split rows finish in the same launch)
-DOMINANT_KERNEL = {"sum": "k_rows<SumOp,4,256,4>", "mean": "k_rows<SumOp,4,256,4>",
-                   "amax": "k_rows<ArgOp<true>,4,256,4>", "argmax": "k_rows<ArgOp<true>,4,256,4>",
-                   "var": "k_rows<WelfordOp,4,256,4>", "std": "k_rows<WelfordOp,4,256,4>"}
+DOMINANT_KERNEL = {"sum": "k_rows<SumOp,256,4>", "mean": "k_rows<SumOp,256,4>",
+                   "amax": "k_rows<ArgOp<true>,256,4>", "argmax": "k_rows<ArgOp<true>,256,4>",
+                   "var": "k_rows<WelfordOp,256,4>", "std": "k_rows<WelfordOp,256,4>"}
 # the C2 strided ops
 C2_KERNEL = {"mean_dim1": "k_cols<SumOp,4,64,4,512>",
              "amax_dim0": "k_cols<ArgOp<true>,4,256,2,256>", "argmax_dim0": "k_cols<ArgOp<true>,4,256,2,256>",
