@@ -2189,10 +2189,16 @@ __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void k_rows_i(Args
 #pragma unroll
             for (int u = 0; u < 4; ++u) acc_vec<Op, T, NV>(acc, t[u], (v + u * step) * NV, prm);
         }
-        for (; v < nv; v += step) {
-            T t[NV];
-            ld16<true>(t, p + (long long)v * NV);
-            acc_vec<Op, T, NV>(acc, t, v * NV, prm);
+        // up to three more, in flight together (int8 [8192, 8192] sums over rows 12.4 ->
+        // 11.1 us, int32 [10, 705, 870] over 2 9.7 -> 8.0)
+        if (v < nv) {
+            T t[3][NV];
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                if (v + u * step < nv) ld16<true>(t[u], p + (long long)(v + u * step) * NV);
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                if (v + u * step < nv) acc_vec<Op, T, NV>(acc, t[u], (v + u * step) * NV, prm);
         }
         for (int e = nv * NV + s * LANES + l; e < R; e += a.S * LANES) Op::acc(acc, p[e], e, prm);
     }
