@@ -2045,7 +2045,7 @@ struct IntArgOp {
     static constexpr bool kIndexed = true;
     static constexpr IdxT kNone = (IdxT)(sizeof(IdxT) == 4 ? 0x7fffffff : kSentinel);
     // 32-bit keys per thread where the values fit: half the instructions per element
-    // ([8192, 8192] uint8 argmax over rows 20.5 -> 17.4 us)
+    // ([8192, 8192] uint8 argmax over rows 20.5 -> 17.0 us)
     using Key = typename std::conditional<(sizeof(T) < 4 || (sizeof(T) == 4 && !IntLimits<T>::U)), int, long long>::type;
     struct Acc { Key v; IdxT i; };
     using State = ArgSI;
@@ -2190,7 +2190,7 @@ __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void k_rows_i(Args
             for (int u = 0; u < 4; ++u) acc_vec<Op, T, NV>(acc, t[u], (v + u * step) * NV, prm);
         }
         // up to three more, in flight together (int8 [8192, 8192] sums over rows 12.4 ->
-        // 11.1 us, int32 [10, 705, 870] over 2 9.7 -> 8.0)
+        // 11.1 us)
         if (v < nv) {
             T t[3][NV];
 #pragma unroll
