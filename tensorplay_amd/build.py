@@ -61,8 +61,8 @@ def _tpr_compiles(force, dev):
     bdir = os.path.join(BUILD, "dev") if dev else BUILD
     os.makedirs(bdir, exist_ok=True)
     inc = ["-I", os.path.join(ROOT, "include"), "-I", os.path.join(CSRC, "rocm")]
-    headers = [os.path.join(ROOT, "include", "tpr_rocm.h"), os.path.join(CSRC, "rocm", "common.h"),
-               os.path.join(CSRC, "rocm", "select.h")]
+    headers = [os.path.join(CSRC, "rocm", h) for h in os.listdir(os.path.join(CSRC, "rocm")) if h.endswith(".h")]
+    headers.append(os.path.join(ROOT, "include", "tpr_rocm.h"))
     extra = ["-DTPR_DEBUG_KNOBS"] if dev else []
     objs, cmds = [], []
     for src in ROCM_SOURCES:
