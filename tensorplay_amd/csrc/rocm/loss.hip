@@ -20,6 +20,7 @@
 #include <string>
 
 #include "common.h"
+#include "nll_walk.h"
 
 namespace tpr {
 namespace {
@@ -221,18 +222,10 @@ __global__ __launch_bounds__(kNllBlock) void k_nll_bwd_short(NllBwdArgs a) {
     const unsigned e = (blockIdx.x * (unsigned)kNllBlock + threadIdx.x) * 4u;
     const unsigned c = (unsigned)a.c, total = (unsigned)(a.n * a.c);
     if (e >= total) return;
-    unsigned row = e / c, col = e - row * c;
-    long long t = a.t[(long long)row * a.ts];
-    f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (t == (long long)col && t != a.ignore) z[k] = nll_grad_value(a, row, t);
-        if (++col == c && e + k + 1 < total) {
-            col = 0;
-            t = a.t[(long long)++row * a.ts];
-        }
-    }
-    nll_store(a.gi, e, total, z);
+    float z[4];
+    nll_short_vector(e, c, total, a.ignore, [&](unsigned i) { return a.t[(long long)i * a.ts]; },
+                     [&](unsigned i, long long t) { return nll_grad_value(a, i, t); }, z);
+    nll_store(a.gi, e, total, f32x4_t{z[0], z[1], z[2], z[3]});
 }
 
 // Short rows beyond 32-bit indices: one element per thread over the

@@ -48,3 +48,21 @@ def test_targets_out_of_range_set_the_flag():
         assert int(_capi.nll_loss(x, t)[2]) == 1
         gi = _capi.nll_loss_backward(torch.ones(1, device="cuda"), t, n, 7, None, 2)
         assert float(gi[n - 1].abs().sum()) == 0 and float(gi.sum()) == -(n - 1)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5])
+@pytest.mark.parametrize("past", [0, 1, 2, 3])
+def test_weighted_target_past_the_last_class(n, past):
+    """The last sample's target c .. c + 3 has no column: its row is all zeros
+    (n * 7 leaves remainders of 1, 2 and 3 to the last vector)."""
+    c = 7
+    print(f"case nll weighted last target c+{past} n={n}", flush=True)
+    w = (torch.arange(c, dtype=torch.float32) + 1).cuda()
+    t = torch.arange(n, dtype=torch.int64) % c
+    t[n - 1] = c + past
+    go = torch.full((1,), 2.0, device="cuda")
+    gi = _capi.nll_loss_backward(go, t.cuda(), n, c, w, 2).cpu()
+    ref = torch.zeros((n, c))
+    for i in range(n - 1):
+        ref[i, t[i]] = -2.0 * float(t[i] + 1)
+    assert torch.equal(gi, ref)
