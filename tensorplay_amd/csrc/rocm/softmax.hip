@@ -2025,9 +2025,10 @@ template <int MODE>
 int run_rows(const SmxArgs& a0, int vw, hipStream_t st) {
     SmxArgs a = a0;
     const int two_pass = knobs().smx_two_pass;
-    // rows off 16 bytes whose output lies over an input keep the kernels that
-    // never read a row again after another workgroup may have written it
-    const bool pieces_ok = vw == 4 || (a.out != a.a && a.out != a.b);
+    // an output that lies over an input keeps the kernels in which one workgroup
+    // reads and writes a row: a piece that recomputes its partner's part reads
+    // input that the partner may have overwritten by then
+    const bool pieces_ok = a.out != a.a && a.out != a.b;
     // gradients: g and y both held (row pieces over workgroups), each read once
     if constexpr (MODE >= BWD) {
         // 512-thread pieces of 24 float4 per lane; measured on MI355X (us):
@@ -2105,7 +2106,7 @@ int run_cols(const SmxColArgs& a_in, hipStream_t st) {
     const bool al16 = a.inner % 4 == 0 && al(a.a) && al(a.out) && a.a_so % 4 == 0 && a.a_sn % 4 == 0 &&
                       (!BW || (al(a.b) && a.b_so % 4 == 0 && a.b_sn % 4 == 0));
     // an output over one of its inputs keeps the kernels in which a column has one
-    // reader and writer, where vectors would share columns
+    // reader and writer: no shared columns, no pieces of a column that are read again
     const bool alias = a.out == a.a || a.out == a.b;
     const bool v4 = a.a_si == 1 && (!BW || a.b_si == 1) && a.inner >= 16 && (al16 || !alias) && knobs().general == 0;
     // vectors off 16 bytes share cache lines, which a nontemporal line may not wait for
@@ -2122,7 +2123,8 @@ int run_cols(const SmxColArgs& a_in, hipStream_t st) {
             if constexpr (!BW) {
                 const long long gp = 2 * blocks;
                 if (a.n > 512 && a.n <= 1024 && knobs().smx_res >= 0 && knobs().smx_two_pass == 0 &&
-                    knobs().smx_fwd_pieces >= 0 && knobs().smx_pieces >= 0 && gp * 128 <= kSmxSlots && !capturing(st)) {
+                    knobs().smx_fwd_pieces >= 0 && knobs().smx_pieces >= 0 && gp * 128 <= kSmxSlots && !alias &&
+                    !capturing(st)) {
                     unsigned ep = smx_epoch_ctr.fetch_add(1, std::memory_order_relaxed) + 1u;
                     if (ep == 0) ep = smx_epoch_ctr.fetch_add(1, std::memory_order_relaxed) + 1u;
                     const int spin = knobs().smx_spin < 0 ? 0 : 4000;
