@@ -1580,10 +1580,15 @@ Plan make_plan(const tpr_reduce_desc* d) {
     };
 
     const long long kIntMax = 0x7fffffffLL;
+    // The row and column kernels count a run's elements in int, and a lane looks up
+    // to one round of all splits past the run's end for its next element: at most
+    // 512 threads per CU times 16 elements (2 M), so runs that come within 2^24 of
+    // 2^31 are cut as well.
+    const long long kRunMax = kIntMax - (1LL << 24);
     const long long kChunk = 1LL << 30;  // elements; a multiple of 16, so chunk starts keep 16-byte alignment
-    if (!empty && !force_general && Rd.size() == 1 && Rd[0].size >= kIntMax) {
+    if (!empty && !force_general && Rd.size() == 1 && Rd[0].size > kRunMax) {
         Rfull = Rd[0].size;
-        Rd[0].size = kChunk;  // plan one chunk; the general kernel takes the whole run back
+        Rd[0].size = kChunk;  // plan one chunk; the run and general kernels take the whole run back
     }
     const bool int_ok = Rd.empty() || (Rd.size() == 1 ? Rd[0].size : p.count) < kIntMax;
     if (empty || force_general || !int_ok) {
@@ -1694,6 +1699,10 @@ Plan make_plan(const tpr_reduce_desc* d) {
         p.S = std::max(1LL, std::min(S, ceil_div(p.R, ty)));
     } else if (!Rd.empty() && Rd.back().stride == 1 && Rd.back().size >= 4 && p.count < kIntMax) {
         // runs: the innermost reduced dim contiguous
+        if (Rfull) {  // cut into units of its own: no chunks
+            Rd[0].size = Rfull;
+            Rfull = 0;
+        }
         p.kind = P_RUNS;
         p.nk = (int)K.size();
         p.nr = (int)Rd.size() - 1;
@@ -1887,8 +1896,8 @@ int launch_finalize(const Plan& p, void* out, const void* ws, Fin fin, hipStream
     return check_launch("k_finalize");
 }
 
-// Launches `launch(plan, in, ws)` once per chunk of a reduced run of 2^31 or
-// more elements: the chunk's input, its R, its index offset and its slice of
+// Launches `launch(plan, in, ws)` once per chunk of a reduced run of nearly 2^31
+// or more elements: the chunk's input, its R, its index offset and its slice of
 // the partial states.  Then one finalize over the S * nchunk partials.
 template <class Op, class Launch>
 int run_chunks(const Plan& p, const void* in, size_t esize, void* out, void* ws, Fin fin, hipStream_t st,

@@ -1,4 +1,4 @@
-"""Reductions whose reduced run has 2^31 or more elements (indices past int32).
+"""Reductions whose reduced run has nearly 2^31 or more elements (indices past int32).
 
 Such runs are cut into chunks of 2^30 elements, one row / column kernel launch
 each, with the chunk's first index added to arg-op states and one finalize over
@@ -89,4 +89,37 @@ def test_float32_full_argmax_past_2_31():
     m = float(red(x, "mean"))
     assert abs(m - 0.5 / N) <= 1e-6 * (0.5 / N)
     del x
+    torch.cuda.empty_cache()
+
+
+def test_runs_just_below_2_31():
+    """Runs that end within 2^24 of 2^31 are cut as well: in one launch the
+    kernels' int indices would pass 2^31 on the way to their next element."""
+    for n in (B - 1, B - 2, B - 100000, B - (1 << 24)):
+        print(f"case int8 full n={n}", flush=True)
+        x = torch.ones(n, dtype=torch.int8, device="cuda")
+        x[n - 1] = 100
+        x[1] = -7
+        assert int(red(x, "sum")) == n - 2 + 100 - 7
+        assert int(red(x, "argmax")) == n - 1
+        assert int(red(x, "argmin")) == 1
+        del x
+    n = B - 3
+    print(f"case float32 full n={n} (8 GiB)", flush=True)
+    y = torch.zeros(n, dtype=torch.float32, device="cuda")
+    y[7] = 3.0
+    y[n - 1] = -4.0
+    assert float(red(y, "sum")) == -1.0
+    assert int(red(y, "argmin")) == n - 1
+    assert _capi.reduce(y, "norm", None, p=2.0).item() == 5.0
+    # powf in the remainder loop; 3^3 + 4^3 = 91, exact in float32 up to powf's rounding (2 ulp each, the root 2 more)
+    v = _capi.reduce(y, "norm", None, p=3.0).item()
+    assert abs(v - 91.0 ** (1 / 3)) <= 6 * 2.0 ** -23 * 91.0 ** (1 / 3)
+    del y
+    print(f"case int8 cols [{n}, 2]", flush=True)
+    z = torch.zeros((n, 2), dtype=torch.int8, device="cuda")
+    z[n - 1, 1] = 9
+    np.testing.assert_array_equal(red(z, "sum", [0]), [0, 9])
+    np.testing.assert_array_equal(red(z, "argmax", [0]), [0, n - 1])
+    del z
     torch.cuda.empty_cache()
