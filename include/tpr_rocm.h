@@ -168,7 +168,8 @@ int tpr_reduce_backward(const tpr_reduce_desc* desc, const void* grad_out, const
  * Order: value descending for largest=1 (ascending for largest=0), equal
  * values by lowest index; -0.0 == +0.0; NaN ranks above every number.
  * sorted=0 is accepted and returns the same (sorted) order.
- * k must satisfy 0 <= k <= cols.  No reference counterpart: TensorPlay has no
+ * k must satisfy 0 <= k <= cols; k above 2^29 and rows longer than 2^31 - 1
+ * are not implemented.  No reference counterpart: TensorPlay has no
  * topk; this adds the schema row
  *   topk(Tensor self, int64_t k, int64_t dim=-1, bool largest=true,
  *        bool sorted=true) -> (Tensor values, Tensor indices)

@@ -95,6 +95,8 @@ constexpr int kWB = 256;                      // per-wave list capacity
 constexpr int kWaveCompact = 192;             // per-wave list size that always triggers compaction
 constexpr int kSlice = 64 * 16;               // elements per wave slice (4 float4 per lane)
 constexpr int kWaveMinSeg = kW * kSlice;      // every wave has a full first slice (8192)
+constexpr long long kIntCols = 0x7fffffffLL - (1LL << 20);  // longest row of the kernels with int indices (route_topk)
+constexpr long long kSortMax = 1LL << 29;     // largest k: the sort's sizes are powers of two in int, and their double
 constexpr long long kWaveMaxSeg = 1LL << 28;  // longest wave-kernel segment (32-bit byte offsets)
 
 // Output value of a selected element: from its key, or from the input row when
@@ -802,7 +804,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(OCC, 8)
     const int k = a.k;
     const int largest = a.largest;
     const int lo = seg * a.seg_len;
-    const int hi = min(a.cols, lo + a.seg_len);
+    const int hi = lo + min(a.cols - lo, a.seg_len);  // lo + seg_len may pass 2^31
     const int nsl = (hi - lo + kSl - 1) / kSl;
     const int r = (k + kW - 1) / kW;
     const int compact_at = min(KWB == kWB ? kWaveCompact : KWB - 64, max(2 * k, 64));  // per-wave list length that triggers compaction
@@ -1074,7 +1076,7 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(6, 8))) void
     const int k = a.k;
     const int largest = a.largest;
     const int lo = seg * a.seg_len;
-    const int hi = min(a.cols, lo + a.seg_len);
+    const int hi = lo + min(a.cols - lo, a.seg_len);  // lo + seg_len may pass 2^31
     const int nchunks = (hi - lo + kCH - 1) / kCH;
     const int r = (k + kW - 1) / kW;
     const int compact_at = max(2 * k, 256);
@@ -2025,12 +2027,13 @@ __device__ int block_suffix_incl(int v, int* wtot) {
 // histogram), then every key > T and the lowest-index keys == T.
 // GB: the gather keeps several loads in flight per thread (more registers).
 template <int NT, class T, bool GB = true>
-__device__ void radix_select(RadixShared<T>& sh, typename Comp<typename SortKey<T>::K>::C* cand, const T* p, int n,
+__device__ void radix_select(RadixShared<T>& sh, typename Comp<typename SortKey<T>::K>::C* cand, const T* p, int n_in,
                              int k, int largest) {
     using K = typename SortKey<T>::K;
     using CP = Comp<K>;
     constexpr int BPT = kRadixBins / NT;  // histogram bins per thread in the digit search
     const int tid = threadIdx.x;
+    const unsigned n = (unsigned)n_in;  // rows of up to 2^31 - 1: an index past the end stays above n
     const int lane = __lane_id();
     const int w = tid / 64;
     K prefix = 0, pmask = 0;
@@ -2042,16 +2045,16 @@ __device__ void radix_select(RadixShared<T>& sh, typename Comp<typename SortKey<
         for (int i = tid; i < kRadixBins; i += NT) sh.hist[i] = 0u;
         __syncthreads();
         // eight loads in flight per thread before their histogram updates
-        int e0 = tid;
+        unsigned e0 = tid;
         for (; e0 + 7 * NT < n; e0 += 8 * NT) {
             K key[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) key[u] = SortKey<T>::of(p[e0 + u * NT], largest);
+            for (int u = 0; u < 8; ++u) key[u] = SortKey<T>::of((p + e0)[u * NT], largest);
 #pragma unroll
             for (int u = 0; u < 8; ++u)
                 if ((key[u] & pmask) == prefix) atomicAdd(&sh.hist[(uint32_t)((key[u] >> shift) & dmask)], 1u);
         }
-        for (int e = e0; e < n; e += NT) {
+        for (unsigned e = e0; e < n; e += NT) {
             const K key = SortKey<T>::of(p[e], largest);
             if ((key & pmask) == prefix) atomicAdd(&sh.hist[(uint32_t)((key >> shift) & dmask)], 1u);
         }
@@ -2090,19 +2093,19 @@ __device__ void radix_select(RadixShared<T>& sh, typename Comp<typename SortKey<
         // GB: GU loads in flight per thread (8 in the 1024-thread kernel, which
         // runs one workgroup per CU anyway; 4 in the 256-thread one)
         constexpr int GU = NT == 1024 ? 8 : 4;
-        int e0 = tid;
+        unsigned e0 = tid;
         for (; GB && e0 + (GU - 1) * NT < n; e0 += GU * NT) {
             K key[GU];
 #pragma unroll
-            for (int u = 0; u < GU; ++u) key[u] = SortKey<T>::of(p[e0 + u * NT], largest);
+            for (int u = 0; u < GU; ++u) key[u] = SortKey<T>::of((p + e0)[u * NT], largest);
 #pragma unroll
             for (int u = 0; u < GU; ++u)
                 if ((key[u] & pmask) >= prefix)
-                    cand[atomicAdd(&sh.count, 1)] = CP::make(key[u], (uint32_t)(e0 + u * NT));
+                    cand[atomicAdd(&sh.count, 1)] = CP::make(key[u], e0 + u * NT);
         }
-        for (int e = e0; e < n; e += NT) {
+        for (unsigned e = e0; e < n; e += NT) {
             const K key = SortKey<T>::of(p[e], largest);
-            if ((key & pmask) >= prefix) cand[atomicAdd(&sh.count, 1)] = CP::make(key, (uint32_t)e);
+            if ((key & pmask) >= prefix) cand[atomicAdd(&sh.count, 1)] = CP::make(key, e);
         }
         __syncthreads();
         return;
@@ -2113,10 +2116,10 @@ __device__ void radix_select(RadixShared<T>& sh, typename Comp<typename SortKey<
         sh.eq_taken = 0;
     }
     __syncthreads();
-    for (int base = 0; base < n; base += NT) {
-        const int e = base + tid;
+    for (unsigned base = 0; base < n; base += NT) {
+        const unsigned e = base + tid;
         const K key = (e < n) ? SortKey<T>::of(p[e], largest) : (K)0;
-        if (e < n && key > Tk) cand[atomicAdd(&sh.count, 1)] = CP::make(key, (uint32_t)e);
+        if (e < n && key > Tk) cand[atomicAdd(&sh.count, 1)] = CP::make(key, e);
         const bool eq = (e < n) && key == Tk;
         const unsigned long long bal = __ballot(eq);
         if (lane == 0) sh.wtot[w] = __popcll(bal);
@@ -2127,15 +2130,15 @@ __device__ void radix_select(RadixShared<T>& sh, typename Comp<typename SortKey<
             if (i < w) before += sh.wtot[i];
             total += sh.wtot[i];
         }
-        if (eq && before < kk) cand[atomicAdd(&sh.count, 1)] = CP::make(key, (uint32_t)e);
+        if (eq && before < kk) cand[atomicAdd(&sh.count, 1)] = CP::make(key, e);
         __syncthreads();
         if (tid == 0) sh.eq_taken += total;
         __syncthreads();
         if (sh.eq_taken >= kk && base + NT < n) {
             // every equal key needed is taken: the rest only adds keys > T
-            for (int e2 = base + NT + tid; e2 < n; e2 += NT) {
+            for (unsigned e2 = base + NT + tid; e2 < n; e2 += NT) {
                 const K k2 = SortKey<T>::of(p[e2], largest);
-                if (k2 > Tk) cand[atomicAdd(&sh.count, 1)] = CP::make(k2, (uint32_t)e2);
+                if (k2 > Tk) cand[atomicAdd(&sh.count, 1)] = CP::make(k2, e2);
             }
             break;
         }
@@ -2759,7 +2762,8 @@ int rsel_segments(long long rows, long long cols, long long k, int32_t dtype) {
 size_t radix_ws(long long rows, long long cols, long long k, int32_t dtype = TPR_FLOAT32) {
     if (rsel_route(cols, k, dtype)) return 0;
     if (const int ns = rsel_segments(rows, cols, k, dtype)) return (size_t)rows * ns * k * sizeof(unsigned long long);
-    const long long n2 = pow2_at_least((int)k);
+    long long n2 = 1;
+    while (n2 < k) n2 <<= 1;
     const bool wide = dtype_size(dtype) == 8;
     const long long lds = wide ? 2048 : kRadixLds;
     return n2 > lds ? (size_t)rows * (size_t)n2 * (wide ? 16 : 8) : 0;
@@ -2790,7 +2794,11 @@ struct TopkRoute {
 // TK_BLOCK with nseg > 1: segment s covers [s * seg_len, min(cols, (s + 1) *
 // seg_len)), every one of the nseg segments holds >= k elements (each writes
 // exactly k composites for the merge), and nseg * k <= kMergeMax.
+// Rows that come within 2^20 elements of 2^31 take the streaming kernel, whose
+// indices are unsigned: the others index past a row's end (a slice, a chunk or
+// the loads in flight) in int before they mask.
 TopkRoute route_topk(long long rows, long long cols, long long k, int32_t dtype, long long row_stride, bool aligned) {
+    if (cols > kIntCols) return TopkRoute{TK_RADIX, 1, (int)cols, 0, radix_ws(rows, cols, k, dtype)};
     const bool radix = radix_route(rows, cols, k, dtype);
     // (The lane-group kernel addresses up to 4 rows per wave with 32-bit offsets.)
     const bool short_ok = (k <= kShortMaxK || short_exact(rows, cols, k)) && cols <= kShortMaxCols &&
@@ -2972,6 +2980,7 @@ int topk_launch(const void* in, int32_t dtype, int64_t rows, int64_t cols, int64
     if (k < 0 || k > cols) return fail(TPR_ERR_INVALID_ARG, "tpr_topk: selected index k out of range");
     if (rows == 0 || k == 0) return TPR_OK;
     if (cols > 0x7fffffffLL) return fail(TPR_ERR_NOT_IMPLEMENTED, "tpr_topk: rows longer than 2^31-1");
+    if (k > kSortMax) return fail(TPR_ERR_NOT_IMPLEMENTED, "tpr_topk: k larger than 2^29");
     if (!in || (!smp && (!out_values || !out_indices))) return fail(TPR_ERR_INVALID_ARG, "tpr_topk: null pointer");
     if (rows > 0x7fffffffLL) return fail(TPR_ERR_NOT_IMPLEMENTED, "tpr_topk: more than 2^31-1 rows");
     const bool aligned = ((reinterpret_cast<uintptr_t>(in) & 15u) == 0) &&
@@ -3155,7 +3164,7 @@ int tpr_topk_plan(int32_t dtype, int64_t rows, int64_t cols, int64_t k, int64_t 
                   int64_t* out) {
     if (!out) return tpr::fail(TPR_ERR_INVALID_ARG, "tpr_topk_plan: null output");
     if (tpr::dtype_size(dtype) == 0) return tpr::fail(TPR_ERR_UNSUPPORTED_DTYPE, "tpr_topk_plan: unknown dtype");
-    if (rows <= 0 || cols <= 0 || k <= 0 || k > cols || cols > 0x7fffffffLL || rows > 0x7fffffffLL)
+    if (rows <= 0 || cols <= 0 || k <= 0 || k > cols || cols > 0x7fffffffLL || rows > 0x7fffffffLL || k > tpr::kSortMax)
         return tpr::fail(TPR_ERR_INVALID_ARG, "tpr_topk_plan: no kernel runs for this shape");
     const tpr::TopkRoute rt = tpr::route_topk(rows, cols, k, dtype, row_stride, aligned != 0);
     out[0] = rt.kind;

@@ -111,3 +111,33 @@ def test_workspace_query_covers_every_alignment():
             for aligned in (True, False):
                 plan_ws = _capi.topk_plan(dtype, rows, cols, k, cols + (0 if aligned else 1), aligned)[4]
                 assert ws >= plan_ws, (dtype, rows, cols, k, aligned, ws, plan_ws)
+
+
+LONGEST = (1 << 31) - 1 - (1 << 20)  # longest row of the kernels whose indices are int
+
+
+@pytest.mark.parametrize("dtype", [_capi.FLOAT32, _capi.INT32, _capi.INT8, _capi.UINT16, _capi.FLOAT64])
+@pytest.mark.parametrize("rows", [1, 3, 300])
+def test_rows_near_2_31_stream(dtype, rows):
+    """Rows within 2^20 of 2^31 elements take the streaming kernel (unsigned
+    indices): the others index a slice or chunk past the row's end in int."""
+    for cols in (LONGEST + 1, (1 << 31) - 16384, (1 << 31) - 1):
+        for k in (1, 50, 128, 300, 1024, 5000):
+            assert _capi.topk_plan(dtype, rows, cols, k)[0] == "radix", (cols, k)
+    kind, nseg = _check(dtype, rows, LONGEST, 50)
+    assert kind != "radix" or dtype == _capi.FLOAT64
+
+
+def test_k_beyond_the_sort_is_refused():
+    """The sort's sizes are powers of two in int: k above 2^29 is refused, and
+    asking for its workspace ends."""
+    L = _capi.lib()
+    big = (1 << 31) - 1
+    for k in ((1 << 29) + 1, 1 << 30, big):
+        assert L.tpr_topk(None, _capi.FLOAT32, 1, big, big, k, 1, 1, None, None, None, 0, None) == _capi.ERR_NOT_IMPLEMENTED
+        with pytest.raises(_capi.TprError):
+            _capi.topk_plan(_capi.FLOAT32, 1, big, k)
+    assert L.tpr_topk_workspace_bytes(_capi.FLOAT32, 1, big, big) == 8 << 31
+    assert L.tpr_sample_workspace_bytes(_capi.FLOAT32, 1, big, big) >= 8 << 31
+    # k = 2^29 is served: the null input is the error
+    assert L.tpr_topk(None, _capi.FLOAT32, 1, big, big, 1 << 29, 1, 1, None, None, None, 0, None) == _capi.ERR_INVALID_ARG
