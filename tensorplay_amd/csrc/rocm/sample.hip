@@ -121,8 +121,8 @@ __device__ __forceinline__ void stream_row(const float* p, int first, int n, F&&
 #pragma unroll
         for (int c = 0; c < 4; ++c) f(v[c], 4 * i + c);
     }
-    const int t = (nv << 2) + threadIdx.x;
-    if (t < n) f(p[t], t);
+    const unsigned t = (unsigned)(nv << 2) + threadIdx.x;  // may pass 2^31
+    if (t < (unsigned)n) f(p[t], (int)t);
 }
 
 __device__ double block_sum(double v, double* sh) {
@@ -244,13 +244,14 @@ __device__ Pick pick(SampleShared& sh, const u64* hist0, const float* p, int n, 
 __device__ void locate(SampleShared& sh, const float* p, int n, uint32_t key, u64 ord, long long* out) {
     const int lane = __lane_id(), w = threadIdx.x >> 6;
     const long long piece = (((long long)n + kNW - 1) / kNW + 63) & ~63ll;
-    const int lo = (int)min((long long)n, w * piece), hi = (int)min((long long)n, (w + 1) * piece);
+    // unsigned: a step past hi may pass 2^31
+    const unsigned lo = (unsigned)min((long long)n, w * piece), hi = (unsigned)min((long long)n, (w + 1) * piece);
     u64 cnt = 0;
-    int b = lo;
+    unsigned b = lo;
     for (; b + 512 <= hi; b += 512) {
         float v[8];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = p[b + q * 64 + lane];
+        for (int q = 0; q < 8; ++q) v[q] = (p + b)[q * 64 + lane];
 #pragma unroll
         for (int q = 0; q < 8; ++q) cnt += (u64)__popcll(__ballot(f2key(v[q], 1) == key));
     }
@@ -550,10 +551,11 @@ __global__ __launch_bounds__(kNT) void k_sample_row(SampleArgs a) {
             if (add(v))
                 for (int c = 0; c < 4; ++c) list(v[c], 4 * i + c);
         }
-        if ((nv << 2) + t < n) {
-            const float v = p[(nv << 2) + t];
+        const unsigned e = (unsigned)(nv << 2) + threadIdx.x;  // may pass 2^31
+        if (e < (unsigned)n) {
+            const float v = p[e];
             if (ALL || f2key(v, 1) > kth) tot += (double)weight(v - v0, a);
-            list(v, (nv << 2) + t);
+            list(v, (int)e);
         }
         double total = block_sum(tot, sh.dsum);
         if (kties) total += (double)kties * (double)weight(__uint_as_float(key2bits(kth, 1)) - v0, a);
