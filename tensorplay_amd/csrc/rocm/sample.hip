@@ -51,6 +51,7 @@ constexpr int kNW = kNT / 64;
 constexpr int kList = 4096;   // candidates sorted in phase 3 (8 per thread)
 constexpr int kListK = 1600;  // largest k tried on a list cut by the bound of phase 2
 constexpr int kBins = 2048;
+constexpr int kUnitRow = 1 << 20;  // rows from here on: draw_by_radix's unit comes from the row's total
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef f4 f4u __attribute__((aligned(4)));  // rows start at any element
@@ -62,9 +63,9 @@ struct SampleArgs {
     long long row_stride;
     int k;
     float temperature, top_p;
+    float scale;       // fixed-point weight of the largest element of a row shorter than kUnitRow (a power of two)
     float c_hi, c_lo;  // log2(e) / temperature as a float pair
     float span;        // temperature * ln(k / (1 - top_p)); < 0: no list
-    float scale;       // fixed-point weight of the largest element (a power of two)
     const float* u;
     long long* ids;
 };
@@ -187,9 +188,10 @@ __device__ void find_digit(SampleShared& sh, const u64* hist, u64 above, u64 tar
     __syncthreads();
 }
 
-// The fixed-point weight of an element; unit: every element weighs 1.
-__device__ __forceinline__ u64 fixed_weight(float v, float v0, bool unit, const SampleArgs& a) {
-    return unit ? 1ull : (u64)(weight(v - v0, a) * a.scale);
+// The fixed-point weight of an element, in units of 1 / scale; unit: every
+// element weighs 1.
+__device__ __forceinline__ u64 fixed_weight(float v, float v0, bool unit, float scale, const SampleArgs& a) {
+    return unit ? 1ull : (u64)(weight(v - v0, a) * scale);
 }
 
 struct Pick {
@@ -198,11 +200,11 @@ struct Pick {
 };
 
 __device__ void first_digit_hist(SampleShared& sh, u64* hist, const float* p, int n, float v0, bool unit,
-                                 const SampleArgs& a) {
+                                 float scale, const SampleArgs& a) {
     for (int i = threadIdx.x; i < kBins; i += kNT) hist[i] = 0;
     __syncthreads();
     stream_row(p, 0, n, [&](float v, int) {
-        const u64 w = fixed_weight(v, v0, unit, a);
+        const u64 w = fixed_weight(v, v0, unit, scale, a);
         if (w) atomicAdd(&hist[f2key(v, 1) >> 21], w);
     });
     __syncthreads();
@@ -210,8 +212,8 @@ __device__ void first_digit_hist(SampleShared& sh, u64* hist, const float* p, in
 
 // The key of the first position whose running weight reaches `target` (1 <=
 // target <= the total weight in hist0, the first digit's histogram).
-__device__ Pick pick(SampleShared& sh, const u64* hist0, const float* p, int n, float v0, bool unit, u64 target,
-                     const SampleArgs& a) {
+__device__ Pick pick(SampleShared& sh, const u64* hist0, const float* p, int n, float v0, bool unit, float scale,
+                     u64 target, const SampleArgs& a) {
     find_digit(sh, hist0, 0, target);
     uint32_t prefix = (uint32_t)sh.digit << 21;
     u64 above = sh.above;
@@ -225,7 +227,7 @@ __device__ Pick pick(SampleShared& sh, const u64* hist0, const float* p, int n, 
         stream_row(p, 0, n, [&](float v, int) {
             const uint32_t key = f2key(v, 1);
             if ((key & pmask) == prefix) {
-                const u64 w = fixed_weight(v, v0, unit, a);
+                const u64 w = fixed_weight(v, v0, unit, scale, a);
                 if (w) atomicAdd(&sh.hist[(key >> shift) & dmask], w);
             }
         });
@@ -279,27 +281,55 @@ __device__ void locate(SampleShared& sh, const float* p, int n, uint32_t key, u6
 
 // Position `target` - 1 in rank order (every element weighs 1).
 __device__ Pick pick_rank(SampleShared& sh, const float* p, int n, u64 target, const SampleArgs& a) {
-    first_digit_hist(sh, sh.hist, p, n, 0.0f, true, a);
-    const Pick r = pick(sh, sh.hist, p, n, 0.0f, true, target, a);
+    first_digit_hist(sh, sh.hist, p, n, 0.0f, true, 0.0f, a);
+    const Pick r = pick(sh, sh.hist, p, n, 0.0f, true, 0.0f, target, a);
     return r;
 }
 
+// The top k's float64 weight that lies on the kties elements of the k-th key.
+__device__ __forceinline__ double ties_weight(float v0, uint32_t kth, u64 kties, const SampleArgs& a) {
+    return kties ? (double)kties * (double)weight(__uint_as_float(key2bits(kth, 1)) - v0, a) : 0.0;
+}
+
 // m and the draw by weighted radix selection over the row in memory.  kth /
-// kties: the k-th key and how many of its elements are among the top k.
+// kties: the k-th key and how many of its elements are among the top k.  total:
+// the top k's float64 weight, below 0 if the caller has not formed it.
+//
+// The unit of the fixed-point weights: an element loses less than one unit to
+// it, a row less than n units.  Rows of fewer than kUnitRow elements leave room
+// for n weights of 1 (a.scale; at most 2^44): a loss below 2^-22 of v_0's weight
+// alone, less than the float32 sums of a sorted row lose.  Longer rows would lose
+// more (2^24 elements: 2^-13 of v_0's weight) and take the unit from their total,
+// which then fills 62 bits: n units are less than 2^(31 - 61) of it.  Where the
+// total has not been formed (top_p = 1) that is one more pass.  LONG is a template
+// parameter: as a test here it cost rows of 10^6 3%.
+template <bool LONG>
 __device__ void draw_by_radix(SampleShared& sh, const float* p, int n, float v0, uint32_t kth, u64 kties, float u,
-                              const SampleArgs& a, long long* out) {
+                              double total_w, const SampleArgs& a, long long* out) {
+    float scale = a.scale;
+    if constexpr (LONG) {
+        if (total_w < 0.0) {
+            double s = 0.0;
+            stream_row(p, 0, n, [&](float v, int) {
+                if (f2key(v, 1) > kth) s += (double)weight(v - v0, a);
+            });
+            total_w = block_sum(s, sh.dsum) + ties_weight(v0, kth, kties, a);
+        }
+        // 1 <= total_w < 2^31: the weights' sum stays below 2^62
+        scale = ldexpf(1.0f, 61 - __builtin_amdgcn_readfirstlane(ilogb(total_w)));
+    }
     // the top k's weights by first digit, and their sum
     for (int i = threadIdx.x; i < kBins; i += kNT) sh.hist0[i] = 0;
     __syncthreads();
     stream_row(p, 0, n, [&](float v, int) {
         const uint32_t key = f2key(v, 1);
         if (key > kth) {
-            const u64 w = fixed_weight(v, v0, false, a);
+            const u64 w = fixed_weight(v, v0, false, scale, a);
             if (w) atomicAdd(&sh.hist0[key >> 21], w);
         }
     });
     if (kties && threadIdx.x == 0) {
-        const u64 w = fixed_weight(__uint_as_float(key2bits(kth, 1)), v0, false, a);
+        const u64 w = fixed_weight(__uint_as_float(key2bits(kth, 1)), v0, false, scale, a);
         if (w) atomicAdd(&sh.hist0[kth >> 21], w * kties);
     }
     __syncthreads();
@@ -316,15 +346,15 @@ __device__ void draw_by_radix(SampleShared& sh, const float* p, int n, float v0,
     __syncthreads();
     const double cut = ceil((double)a.top_p * (double)total);
     const u64 t1 = a.top_p >= 1.0f ? total : min(total, max((u64)1, (u64)cut));
-    const Pick m = pick(sh, sh.hist0, p, n, v0, false, t1, a);
-    const u64 wm = fixed_weight(__uint_as_float(key2bits(m.key, 1)), v0, false, a);
+    const Pick m = pick(sh, sh.hist0, p, n, v0, false, scale, t1, a);
+    const u64 wm = fixed_weight(__uint_as_float(key2bits(m.key, 1)), v0, false, scale, a);
     const u64 ties = (t1 - m.above + wm - 1) / wm;
     const u64 cm = m.above + ties * wm;
     const double thr = (double)u * (double)cm;
     // the first c_j > thr; u >= 1 or NaN leaves m
     const u64 t2 = thr < (double)cm ? (thr < 0.0 ? 1ull : min(cm, (u64)thr + 1ull)) : cm;
-    const Pick d = pick(sh, sh.hist0, p, n, v0, false, t2, a);
-    const u64 wd = fixed_weight(__uint_as_float(key2bits(d.key, 1)), v0, false, a);
+    const Pick d = pick(sh, sh.hist0, p, n, v0, false, scale, t2, a);
+    const u64 wd = fixed_weight(__uint_as_float(key2bits(d.key, 1)), v0, false, scale, a);
     locate(sh, p, n, d.key, (t2 - d.above + wd - 1) / wd, out);
 }
 
@@ -405,8 +435,9 @@ __device__ bool draw_from_list(SampleShared& sh, int cnt, int k, float v0, doubl
 
 // VR float4 of the row per thread in registers (the host picks VR with VR * 4 *
 // kNT <= cols, so the register part needs no range checks).  ALL: k = cols (no
-// k-th key; the test per element on it costs registers and time).
-template <int VR, bool ALL>
+// k-th key; the test per element on it costs registers and time).  LONG: rows of
+// kUnitRow elements or more.
+template <int VR, bool ALL, bool LONG = false>
 __global__ __launch_bounds__(kNT) void k_sample_row(SampleArgs a) {
     __shared__ SampleShared sh;
     const long long row = blockIdx.x;
@@ -492,6 +523,7 @@ __global__ __launch_bounds__(kNT) void k_sample_row(SampleArgs a) {
         kth = r.key;
         kties = (u64)a.k - r.above;
     }
+    double total = -1.0;
     if (a.span >= 0.0f) {
         // 2. the top k's total weight and the elements at or above the bound
         float bound = v0 - a.span;
@@ -557,8 +589,8 @@ __global__ __launch_bounds__(kNT) void k_sample_row(SampleArgs a) {
             if (ALL || f2key(v, 1) > kth) tot += (double)weight(v - v0, a);
             list(v, (int)e);
         }
-        double total = block_sum(tot, sh.dsum);
-        if (kties) total += (double)kties * (double)weight(__uint_as_float(key2bits(kth, 1)) - v0, a);
+        total = block_sum(tot, sh.dsum);
+        total += ties_weight(v0, kth, kties, a);
         const int cnt = sh.count;
         __syncthreads();
         if (cnt <= kList) {
@@ -566,7 +598,7 @@ __global__ __launch_bounds__(kNT) void k_sample_row(SampleArgs a) {
             __syncthreads();
         }
     }
-    draw_by_radix(sh, p, n, v0, kth, kties, u, a, &a.ids[row]);
+    draw_by_radix<LONG>(sh, p, n, v0, kth, kties, u, total, a, &a.ids[row]);
 }
 
 }  // namespace
@@ -593,8 +625,11 @@ int sample_rows(const float* in, long long rows, long long cols, long long row_s
     a.ids = ids;
     const dim3 g((unsigned)rows), b(kNT);
     const long long per = cols / (4 * kNT);  // whole vectors per thread
-#define TPR_SAMPLE(VR, ALL) hipLaunchKernelGGL((k_sample_row<VR, ALL>), g, b, 0, st, a)
-    if (k < cols) TPR_SAMPLE(0, false);
+#define TPR_SAMPLE(...) hipLaunchKernelGGL((k_sample_row<__VA_ARGS__>), g, b, 0, st, a)
+    if (cols >= kUnitRow) {
+        if (k < cols) TPR_SAMPLE(0, false, true);
+        else TPR_SAMPLE(54, true, true);
+    } else if (k < cols) TPR_SAMPLE(0, false);
     else if (per >= 54) TPR_SAMPLE(54, true);
     else if (per >= 36) TPR_SAMPLE(36, true);
     else if (per >= 24) TPR_SAMPLE(24, true);
