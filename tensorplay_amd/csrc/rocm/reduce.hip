@@ -2145,6 +2145,31 @@ __device__ __forceinline__ void ld16(T (&t)[NV], const T* p) {
     __builtin_memcpy(&t, &w, 16);
 }
 
+// Sums of narrow integers: the extension to register pairs makes the compiler copy
+// one load's elements before it issues the next predicated load, one wait for each
+// load (int32 [300, 1500, 100] over 2: 39.0 us, a rolled loop 36.2).  There the
+// loads are not predicated, and a use of all three holds them together (32.0).  The
+// other ops' predicated loads go out together as they are, and lose to the extra
+// loads (int32 argmax 30.7 -> 32.5).
+template <class Op, class T>
+constexpr bool kHoldTail = std::is_same<Op, IntSumOp<T, false>>::value && sizeof(T) <= 4;
+template <class Op, class T>
+constexpr bool kHoldVec = kHoldTail<Op, T> && sizeof(T) >= 2;  // bytes are added four at a time, not extended
+
+// A use of three loaded vectors at once, behind all three loads.
+template <class T, int NV>
+__device__ __forceinline__ void hold16(T (&a)[NV], T (&b)[NV], T (&c)[NV]) {
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    i32x4 x, y, z;
+    __builtin_memcpy(&x, &a, 16);
+    __builtin_memcpy(&y, &b, 16);
+    __builtin_memcpy(&z, &c, 16);
+    __asm__ volatile("" : "+v"(x), "+v"(y), "+v"(z));
+    __builtin_memcpy(&a, &x, 16);
+    __builtin_memcpy(&b, &y, 16);
+    __builtin_memcpy(&c, &z, 16);
+}
+
 template <class Op, int LANES>
 __device__ __forceinline__ typename Op::State combine_lanes(typename Op::State st, int tid) {
     using State = typename Op::State;
@@ -2186,7 +2211,28 @@ __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void k_rows_i(Args
     if (row < a.rows) {
         const T* p = static_cast<const T*>(a.in) + row * a.row_stride;
         const int R = (int)a.R;
-        const int nv = R / NV;
+        // short rows of 1- and 2-byte elements (16 lanes): one element per lane and
+        // load; few lanes would hold a vector (int8 [400000, 31] sums 15.9 -> 12.6 us)
+        const bool few = LANES == 16 && sizeof(T) <= 2 && R >= NV && R < 32;
+        const int nv = few ? 0 : R / NV;
+        if constexpr (LANES == 16 && sizeof(T) <= 2) {
+            if (few && s == 0 && l < R) {
+                const T x0 = p[l], x1 = p[min(l + 16, R - 1)];
+                Op::acc(acc, x0, l, prm);
+                if (l + 16 < R) Op::acc(acc, x1, l + 16, prm);
+            }
+        }
+        // the last R % NV elements (fewer than 16): one each for the first lanes, loaded
+        // first (after the vectors: float64 [400000, 31] sums 27.5 us, so 22.0; int8
+        // [450000, 100] 26.0 and 19.6)
+        const int te = nv * NV + l;
+        bool tail = false;
+        T xt = T(0);
+        if (__builtin_expect((R & (NV - 1)) != 0, 0)) {
+            tail = s == 0 && te < R && !few;
+            if constexpr (kHoldTail<Op, T>) xt = p[min(te, R - 1)];
+            else if (tail) xt = p[te];
+        }
         const int step = a.S * LANES;
         int v = s * LANES + l;
         // four vectors in flight per lane; each lane still visits its
@@ -2200,16 +2246,34 @@ __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void k_rows_i(Args
         }
         // up to three more, in flight together (int8 [8192, 8192] sums over rows 12.4 ->
         // 11.1 us)
-        if (v < nv) {
-            T t[3][NV];
+        const bool more = v < nv;
+        T t[3][NV];
+        if (more) {
+            if constexpr (kHoldVec<Op, T>) {
+                if (step < nv) {  // past the row's end the last vector again, not accumulated
 #pragma unroll
-            for (int u = 0; u < 3; ++u)
-                if (v + u * step < nv) ld16<true>(t[u], p + (long long)(v + u * step) * NV);
+                    for (int u = 0; u < 3; ++u) ld16<true>(t[u], p + (long long)min(v + u * step, nv - 1) * NV);
+                    hold16(t[0], t[1], t[2]);
+                } else {
+                    ld16<true>(t[0], p + (long long)v * NV);
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < 3; ++u)
+                    if (v + u * step < nv) ld16<true>(t[u], p + (long long)(v + u * step) * NV);
+            }
+        }
+        if (more) {
 #pragma unroll
             for (int u = 0; u < 3; ++u)
                 if (v + u * step < nv) acc_vec<Op, T, NV>(acc, t[u], (v + u * step) * NV, prm);
         }
-        for (int e = nv * NV + s * LANES + l; e < R; e += a.S * LANES) Op::acc(acc, p[e], e, prm);
+        if constexpr (kHoldTail<Op, T>) {
+            int x = (int)xt;
+            __asm__ volatile("" : "+v"(x));
+            xt = (T)x;
+        }
+        if (tail) Op::acc(acc, xt, te, prm);
     }
     using State = typename Op::State;
     State st = combine_lanes<Op, LANES>(Op::state(acc), tid);
