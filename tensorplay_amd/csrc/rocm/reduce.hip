@@ -1529,8 +1529,9 @@ Plan make_plan(const tpr_reduce_desc* d) {
     for (auto& x : dims) (x.red ? Rd : K).push_back(x);
     // Where the result does not depend on the order of the reduced elements
     // (not argmax/argmin, nor the sign of a zero extremum of a float amax/amin)
-    // the reduced dims are visited in memory order, whatever the view's.
-    const bool ordered = d->op == TPR_ARGMAX || d->op == TPR_ARGMIN ||
+    // the reduced dims are visited in memory order, whatever the view's.  Nor the
+    // median's: it takes views that are contiguous as they stand, and refuses others.
+    const bool ordered = d->op == TPR_ARGMAX || d->op == TPR_ARGMIN || d->op == TPR_MEDIAN ||
                          ((d->op == TPR_AMAX || d->op == TPR_AMIN || d->op == TPR_NORM) &&
                           (d->in_dtype == TPR_FLOAT32 || d->in_dtype == TPR_FLOAT64));
     if (!ordered) {

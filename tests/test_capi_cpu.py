@@ -160,3 +160,15 @@ def test_softmax_loss_validation_without_gpu():
     assert L.tpr_nll_loss(*args) == _capi.ERR_WORKSPACE
     assert L.tpr_nll_loss_backward(None, 1, None, 1, None, None, 0, 5, 1, -100, None, None) == _capi.OK
     assert L.tpr_nll_loss_backward(None, 1, None, 1, None, None, 2, 5, 4, -100, None, None) == _capi.ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("dt", [_capi.FLOAT32, _capi.FLOAT64, _capi.INT16])
+def test_median_of_a_permuted_view_is_refused_without_gpu(dt):
+    """Only a view that is contiguous in its own order is served."""
+    L = _capi.lib()
+    for sizes, strides in (([4, 6], [1, 4]), ([2, 3, 4], [1, 2, 6]), ([5, 6], [12, 2])):
+        d = _capi.make_desc("median", sizes, strides, list(range(len(sizes))), dt, in_dtype=dt)
+        assert L.tpr_reduce(ctypes.byref(d), 16, 16, None, 0, None) == _capi.ERR_NOT_IMPLEMENTED
+        assert b"contiguous" in L.tpr_last_error()
+    d = _capi.make_desc("median", [4, 6], [6, 1], [0, 1], dt, in_dtype=dt)
+    assert L.tpr_reduce(ctypes.byref(d), 16, 16, None, 0, None) == _capi.ERR_WORKSPACE  # served: the workspace is missing
