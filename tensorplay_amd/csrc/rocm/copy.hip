@@ -567,7 +567,9 @@ int launch_copy(const CopyPlan& p, void* dst, const void* src, hipStream_t st) {
         a.L = p.dims.back().size;
         a.chunk = kCopyBlock * (16 / (long long)sizeof(D));
         a.nchunk = (a.L + a.chunk - 1) / a.chunk;
-        if (fits && a.nchunk <= 0x7fffffffLL && rows * a.nchunk <= 0x7fffffffLL) {
+        // a launch counts its threads in 32 bits; k_copy_elem strides over any size
+        constexpr long long kMaxBlocks = 0xffffffffLL / kCopyBlock;
+        if (fits && a.nchunk <= kMaxBlocks && rows * a.nchunk <= kMaxBlocks) {
             hipLaunchKernelGGL((k_copy_srows<D, S>), dim3((unsigned)(rows * a.nchunk)), dim3(kCopyBlock), 0, st, a,
                                p.dims.back().ss);
             return check_launch("k_copy_srows");
