@@ -13,6 +13,10 @@ namespace tpr {
 
 constexpr int kWave = 64;  // CDNA wavefront width
 
+// A launch counts its threads in 32 bits: a larger one runs what is left of them
+// modulo 2^32 and reports no error, so launches stay below this.
+constexpr long long kMaxThreads = 0xffffffffLL;
+
 // ---- error plumbing (host) -------------------------------------------------
 void set_error(const std::string& msg);
 int fail(int status, const std::string& msg);

@@ -1729,6 +1729,21 @@ Plan make_plan(const tpr_reduce_desc* d) {
     return p;
 }
 
+// Threads of the plan's launch.
+long long plan_threads(const Plan& p) {
+    switch (p.kind) {
+        case P_ROWS: {
+            if (p.reg_wpr > 0) return p.rows * p.reg_wpr * kWave + 512;  // whole workgroups
+            const long long groups = p.lanes >= kBlock ? 1 : kBlock / p.lanes;
+            return ceil_div(p.rows, groups) * p.S * std::max(p.lanes, kBlock);
+        }
+        case P_COLS: return p.outer * p.ncb * p.S * p.colblock;
+        case P_RUNS: return p.nout * p.S * p.colblock;
+        case P_FEW_COLS: return p.outer * p.S * kBlock;
+        default: return p.nout * p.S * kBlock;
+    }
+}
+
 // Ops for which an element equal to 0 changes nothing (k_rows_reg reads 0 past a row's end).
 template <class Op>
 constexpr bool kZeroIdentity = std::is_same<Op, SumOp>::value || std::is_same<Op, NormOp<1>>::value ||
@@ -3069,6 +3084,23 @@ int tpr_reduce(const tpr_reduce_desc* desc, const void* in, void* out, void* wor
     if (p.ws > 0 && (workspace == nullptr || workspace_bytes < p.ws))
         return fail(TPR_ERR_WORKSPACE, "tpr_reduce: workspace too small (need " +
                                            std::to_string(p.ws) + " bytes)");
+    if (plan_threads(p) > kMaxThreads && p.nout > 1) {
+        // Hundreds of millions of short rows, tens of millions of other outputs: the
+        // first kept dim in two halves, whose outputs follow each other.  Either has
+        // outputs enough to need no workspace of its own.
+        int i = 0;
+        while (((desc->reduce_mask >> i) & 1u) || desc->sizes[i] == 1) ++i;
+        const long long n = desc->sizes[i], half = n / 2;
+        const long long oe = desc->out_dtype == TPR_FLOAT32 ? 4 : esize_of(desc->out_dtype);
+        const long long ie = int_in ? esize_of(desc->in_dtype) : 4;
+        tpr_reduce_desc part = *desc;
+        part.sizes[i] = half;
+        rc = tpr_reduce(&part, in, out, workspace, workspace_bytes, stream);
+        if (rc != TPR_OK) return rc;
+        part.sizes[i] = n - half;
+        return tpr_reduce(&part, static_cast<const char*>(in) + half * desc->strides[i] * ie,
+                          static_cast<char*>(out) + half * (p.nout / n) * oe, workspace, workspace_bytes, stream);
+    }
     Fin fin;
     fin.op = desc->op;
     fin.out_f64 = desc->out_dtype == TPR_FLOAT64;
