@@ -461,10 +461,43 @@ CopyPlan plan_copy(const tpr_copy_desc* d, void* dst, const void* src) {
     return p;
 }
 
+// Workgroups of the plan's launch (0: a kernel that strides over any size).
+template <class D, class S>
+long long copy_blocks(const CopyPlan& p) {
+    const long long V = 16 / (long long)sizeof(S);
+    if (p.kind == C_CONTIG) return p.vec ? (p.n + kCopyBlock * V * kChunkVecs - 1) / (kCopyBlock * V * kChunkVecs) : 0;
+    if (p.kind == C_ROWS) {
+        const long long L = p.dims.back().size, chunk = kCopyBlock * V * kChunkVecs;
+        return p.n / L * ((L + chunk - 1) / chunk);
+    }
+    if (p.kind == C_TILE) {
+        const long long I = p.dims.back().size, J = p.dims[p.J].size;
+        return p.n / (I * J) * ((I + kTile - 1) / kTile) * ((J + kTile - 1) / kTile);  // its tiles are this or larger
+    }
+    return 0;
+}
+
 template <class D, class S>
 int launch_copy(const CopyPlan& p, void* dst, const void* src, hipStream_t st) {
     const auto& dev = device_info();
     const int nd = (int)p.dims.size();
+    if (copy_blocks<D, S>(p) > kMaxThreads / kCopyBlock) {
+        // more than one launch's threads (64 GiB of dense data): the outermost dim in
+        // two parts, the first of whole vectors where vectors run along it
+        int i = 0;
+        while (i + 1 < nd && p.dims[i].size == 1) ++i;
+        const long long n = p.dims[i].size, half = n >= 256 ? (n / 2) & ~127LL : n / 2;
+        CopyPlan h = p;
+        if (half & 15) h.vec = p.vec && i != p.J && i + 1 != nd;
+        h.dims[i].size = half;
+        h.n = p.n / n * half;
+        const int rc = launch_copy<D, S>(h, dst, src, st);
+        if (rc != TPR_OK) return rc;
+        h.dims[i].size = n - half;
+        h.n = p.n / n * (n - half);
+        return launch_copy<D, S>(h, static_cast<D*>(dst) + half * p.dims[i].ds,
+                                 static_cast<const S*>(src) + half * p.dims[i].ss, st);
+    }
     if (p.kind == C_CONTIG) {
         const long long bytes = p.n * (long long)(sizeof(D) + sizeof(S));
         ContigArgs a{dst, src, p.n};
@@ -568,7 +601,7 @@ int launch_copy(const CopyPlan& p, void* dst, const void* src, hipStream_t st) {
         a.chunk = kCopyBlock * (16 / (long long)sizeof(D));
         a.nchunk = (a.L + a.chunk - 1) / a.chunk;
         // a launch counts its threads in 32 bits; k_copy_elem strides over any size
-        constexpr long long kMaxBlocks = 0xffffffffLL / kCopyBlock;
+        constexpr long long kMaxBlocks = kMaxThreads / kCopyBlock;
         if (fits && a.nchunk <= kMaxBlocks && rows * a.nchunk <= kMaxBlocks) {
             hipLaunchKernelGGL((k_copy_srows<D, S>), dim3((unsigned)(rows * a.nchunk)), dim3(kCopyBlock), 0, st, a,
                                p.dims.back().ss);
