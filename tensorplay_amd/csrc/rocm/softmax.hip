@@ -1055,6 +1055,7 @@ struct SmxColArgs {
     long long a_so, a_sn, a_si;
     long long b_so, b_sn, b_si;
     int nt;  // nontemporal second-pass loads and stores
+    long long col0 = 0;  // k_smx_cols: first column of the launch
 };
 
 template <int MODE, int BY>
@@ -1066,7 +1067,7 @@ __global__ __launch_bounds__(kWave * BY) void k_smx_cols(SmxColArgs p) {
     const int lane = threadIdx.x % kWave;
     const int w = threadIdx.x / kWave;
     const long long cols = p.outer * p.inner;
-    const long long col = (long long)blockIdx.x * kWave + lane;
+    const long long col = p.col0 + (long long)blockIdx.x * kWave + lane;
     const bool live = col < cols;
     const long long o = live ? col / p.inner : 0;
     const long long i = live ? col - o * p.inner : 0;
@@ -1834,7 +1835,14 @@ template <int MODE>
 int run_f64(const SmxF64Args& a, hipStream_t st) {
     const long long cols = a.outer * a.inner;
     if (a.inner == 1 && a.a_sn == 1 && (MODE < BWD || a.b_sn == 1)) {
-        hipLaunchKernelGGL((k_smx_f64_rows<MODE, true>), dim3((unsigned)a.outer), dim3(256), 0, st, a);
+        const long long most = kMaxThreads / 256;  // rows of one launch
+        for (long long r = 0; r < a.outer; r += most) {
+            SmxF64Args h = a;
+            h.a += r * a.a_so;
+            if (MODE >= BWD) h.b += r * a.b_so;
+            h.out += r * a.n;
+            hipLaunchKernelGGL((k_smx_f64_rows<MODE, true>), dim3((unsigned)std::min(most, a.outer - r)), dim3(256), 0, st, h);
+        }
     } else if (cols < 64LL * device_info().cus && a.n >= 256) {
         // fewer slices than 64 per CU: a workgroup per slice instead of a thread
         hipLaunchKernelGGL((k_smx_f64_rows<MODE, false>), dim3((unsigned)cols), dim3(256), 0, st, a);
@@ -2025,6 +2033,23 @@ template <int MODE>
 int run_rows(const SmxArgs& a0, int vw, hipStream_t st) {
     SmxArgs a = a0;
     const int two_pass = knobs().smx_two_pass;
+    // threads per row, at most: the lane groups of rows_single, else a workgroup
+    // (pieces and chunks of a row are for far fewer rows)
+    const long long q = (a.n + 3) / 4;
+    const long long per = two_pass || q > 1024 ? 1024 : q > 256 ? 256 : q > 64 ? 64 : 16;
+    const long long most = kMaxThreads / per & ~1023LL;  // rows of one launch
+    if (a.rows > most) {
+        for (long long r = 0; r < a0.rows; r += most) {
+            a = a0;
+            a.rows = std::min(most, a0.rows - r);
+            a.a += r * a.sa;
+            if (MODE >= BWD) a.b += r * a.sb;
+            a.out += r * a.n;
+            const int rc = run_rows<MODE>(a, vw, st);
+            if (rc != TPR_OK) return rc;
+        }
+        return TPR_OK;
+    }
     // an output that lies over an input keeps the kernels in which one workgroup
     // reads and writes a row: a piece that recomputes its partner's part reads
     // input that the partner may have overwritten by then
@@ -2113,7 +2138,22 @@ int run_cols(const SmxColArgs& a_in, hipStream_t st) {
     if (!al16 && knobs().nt == 0) a.nt = 0;
     if (v4) {
         const long long blocks = a.outer * ((a.inner + 63) / 64);
-        if (blocks <= 0x7fffffffLL) {
+        // waves per workgroup, at most
+        const long long by = a.n <= 16 && knobs().smx_two_pass == 0 && knobs().smx_res >= 0 ? 1 : a.n <= 256 ? 8 : 16;
+        const long long most = kMaxThreads / (kWave * by);  // workgroups of one launch
+        if (blocks > most && a.outer > 1) {
+            const long long half = a.outer / 2;
+            SmxColArgs h = a_in;
+            h.outer = half;
+            const int rc = run_cols<MODE>(h, st);
+            if (rc != TPR_OK) return rc;
+            h.outer = a.outer - half;
+            h.a += half * a.a_so;
+            if (BW) h.b += half * a.b_so;
+            h.out += half * a.n * a.inner;
+            return run_cols<MODE>(h, st);
+        }
+        if (blocks <= most) {
             // more waves along longer dims (measured at [64, 1024, 1024] dim 1: 16 waves 150 us,
             // 8 waves 160 us; at [16, 256, 8192] dim 1: 8 waves 70 us, 16 waves 92 us)
             // slices of 65..1024 rows (backward, two inputs: ..256) stay in
@@ -2193,11 +2233,16 @@ int run_cols(const SmxColArgs& a_in, hipStream_t st) {
         }
     }
     const long long cols = a.outer * a.inner;
-    const long long blocks = (cols + kWave - 1) / kWave;
-    if (blocks > 0x7fffffffLL) return fail(TPR_ERR_INVALID_ARG, "tpr_softmax: too many slices");
-    if (a.n >= 256) hipLaunchKernelGGL((k_smx_cols<MODE, 8>), dim3((unsigned)blocks), dim3(kWave * 8), 0, st, a);
-    else hipLaunchKernelGGL((k_smx_cols<MODE, 4>), dim3((unsigned)blocks), dim3(kWave * 4), 0, st, a);
-    return check_launch("tpr_softmax (strided dim)");
+    const int by = a.n >= 256 ? 8 : 4;
+    const long long most = kMaxThreads / (kWave * by);  // workgroups of one launch
+    for (a.col0 = 0; a.col0 < cols; a.col0 += most * kWave) {
+        const unsigned blocks = (unsigned)std::min(most, (cols - a.col0 + kWave - 1) / kWave);
+        if (by == 8) hipLaunchKernelGGL((k_smx_cols<MODE, 8>), dim3(blocks), dim3(kWave * 8), 0, st, a);
+        else hipLaunchKernelGGL((k_smx_cols<MODE, 4>), dim3(blocks), dim3(kWave * 4), 0, st, a);
+        const int rc = check_launch("tpr_softmax (strided dim)");
+        if (rc != TPR_OK) return rc;
+    }
+    return TPR_OK;
 }
 
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
