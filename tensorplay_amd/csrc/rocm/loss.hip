@@ -303,7 +303,15 @@ extern "C" int tpr_nll_loss_backward(const void* grad_output, int64_t gs, const 
                  n, c, reduction, ignore_index, static_cast<float*>(grad_input)};
     if (c >= 1024) {
         const long long blocks = (n * c + 4 * kNllBlock - 1) / (4 * kNllBlock);
-        if (blocks > 0x7fffffffLL) return fail(TPR_ERR_INVALID_ARG, "tpr_nll_loss_backward: too large");
+        if (blocks > kMaxThreads / kNllBlock && n > 1) {  // 64 GiB of gradient: the samples in two halves
+            const int64_t h = n / 2;
+            const int rc = tpr_nll_loss_backward(grad_output, gs, target, ts, weight, total_weight, h, c, reduction,
+                                                 ignore_index, grad_input, stream);
+            if (rc != TPR_OK) return rc;
+            return tpr_nll_loss_backward(a.g + (reduction == 0 ? h * gs : 0), gs, target + h * ts, ts, weight, total_weight,
+                                         n - h, c, reduction, ignore_index, a.gi + h * c, stream);
+        }
+        if (blocks > kMaxThreads / kNllBlock) return fail(TPR_ERR_INVALID_ARG, "tpr_nll_loss_backward: too large");
         hipLaunchKernelGGL(k_nll_bwd_rows, dim3((unsigned)blocks), dim3(kNllBlock), 0, st, a);
     } else if (n * c < 0x100000000LL - 4 * kNllBlock) {
         const unsigned blocks = (unsigned)((n * c + 4 * kNllBlock - 1) / (4 * kNllBlock));

@@ -393,7 +393,7 @@ bool launch_vs_cols(const RbArgs& a, hipStream_t st) {
     if (!al(a.x) || !al(a.gi) || b.xs[1] % 4 != 0 || b.xs[0] % 4 != 0) return false;
     const long long ncg = (inner + 63) / 64;
     const long long blocks = outer * ncg;
-    if (blocks > 0x7fffffffLL) return false;
+    if (blocks > kMaxThreads / 1024) return false;
     const dim3 gr((unsigned)blocks);
     if (R <= 128) hipLaunchKernelGGL((k_vs_bwd_cols<OP, 8, 4>), gr, dim3(512), 0, st, b, outer, (int)R, inner, ncg);
     else if (R <= 256) hipLaunchKernelGGL((k_vs_bwd_cols<OP, 8, 8>), gr, dim3(512), 0, st, b, outer, (int)R, inner, ncg);
@@ -420,7 +420,7 @@ bool launch_vs_rows(const RbArgs& a, hipStream_t st) {
         if (a.xs[d] % 4 != 0) return false;  // every row start 16-byte aligned
     const long long rows = a.total / L;
     const long long blocks = (rows + 3) / 4;
-    if (blocks > 0x7fffffffLL) return false;
+    if (blocks > kMaxThreads / 256) return false;
     const int v = L <= 256 ? 1 : L <= 512 ? 2 : L <= 1024 ? 4 : L <= 2048 ? 8 : 16;
     const dim3 gr((unsigned)blocks), bl(256);
     switch (v) {
@@ -470,7 +470,7 @@ int launch_bwd(const RbArgs& a_in, long long nout, hipStream_t st) {
         const long long rows = a.total / L;
         const int rpb = L < ch ? (int)(ch / L) : 1;  // short rows: several per workgroup
         const long long blocks = (rows + rpb - 1) / rpb * chunks;
-        if (blocks <= 0x7fffffffLL) {
+        if (blocks <= kMaxThreads / 256) {  // else k_red_bwd, which strides over any size
             const dim3 gr((unsigned)blocks), bl(256);
 #define TPR_RB_ROWS(VV, II)                                                                                 \
     if (u == 4) hipLaunchKernelGGL((k_red_bwd_rows<OP, VV, II, 4>), gr, bl, 0, st, a, chunks, rpb, rows);     \
