@@ -605,6 +605,13 @@ __global__ __launch_bounds__(kNT) void k_sample_row(SampleArgs a) {
 
 int sample_rows(const float* in, long long rows, long long cols, long long row_stride, long long k, float temperature,
                 float top_p, const float* u, long long* ids, hipStream_t st) {
+    const long long most = kMaxThreads / kNT;  // rows of one launch
+    if (rows > most) {
+        const int rc = sample_rows(in, most, cols, row_stride, k, temperature, top_p, u, ids, st);
+        if (rc != TPR_OK) return rc;
+        return sample_rows(in + most * row_stride, rows - most, cols, row_stride, k, temperature, top_p, u + most,
+                           ids + most, st);
+    }
     SampleArgs a;
     a.in = in;
     a.cols = (int)cols;

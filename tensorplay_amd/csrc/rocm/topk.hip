@@ -2969,6 +2969,18 @@ int launch_rsel(const TopkArgs& a, int32_t dtype, hipStream_t st) {
     return launch_rsel_p<1024, 32>(a, dtype, st);
 }
 
+// Threads that a route's largest launch takes per row, at most.
+long long row_threads(const TopkRoute& rt, long long rows, long long cols) {
+    switch (rt.kind) {
+        case TK_SHORT: case TK_SHORT_SMALL: return 64;
+        case TK_RSEL: return cols <= 4096 ? 256 : cols <= 8192 ? 512 : 1024;
+        case TK_RADIX: return rows < 2LL * device_info().cus ? 1024 : kRadixT;
+        case TK_WAVE: case TK_WAVE8: return std::max(rt.nseg * rt.nw * 64, kRadixT);
+        case TK_BLOCK: return rt.nseg * kT;
+        default: return rt.nseg * 1024LL;
+    }
+}
+
 // tpr_topk, or (smp != nullptr) tpr_sample: the same selection with the draw
 // in the final phase.
 int topk_launch(const void* in, int32_t dtype, int64_t rows, int64_t cols, int64_t row_stride, int64_t k,
@@ -2989,6 +3001,24 @@ int topk_launch(const void* in, int32_t dtype, int64_t rows, int64_t cols, int64
     if (rows * (long long)rt.nseg > 0x7fffffffLL) return fail(TPR_ERR_NOT_IMPLEMENTED, "tpr_topk: grid too large");
     if (rt.ws > 0 && (workspace == nullptr || workspace_bytes < rt.ws))
         return fail(TPR_ERR_WORKSPACE, "tpr_topk: workspace too small (need " + std::to_string(rt.ws) + " bytes)");
+    if (rows * row_threads(rt, rows, cols) > kMaxThreads) {
+        // tens of millions of rows: in two halves, which plan alike and need less workspace
+        const int64_t h = rows / 2;
+        const long long es = dtype_size(dtype);
+        TopkArgs second{};
+        if (smp) {
+            second = *smp;
+            second.u += h;
+            second.ids += h;
+        }
+        const int rc = topk_launch(in, dtype, h, cols, row_stride, k, largest, out_values, out_indices, workspace,
+                                   workspace_bytes, stream, smp);
+        if (rc != TPR_OK) return rc;
+        return topk_launch(static_cast<const char*>(in) + h * row_stride * es, dtype, rows - h, cols, row_stride, k,
+                           largest, smp ? nullptr : static_cast<char*>(out_values) + h * k * es,
+                           smp ? nullptr : static_cast<long long*>(out_indices) + h * k, workspace, workspace_bytes,
+                           stream, smp ? &second : nullptr);
+    }
     TopkArgs a;
     a.in = static_cast<const float*>(in);
     a.rows = rows;
