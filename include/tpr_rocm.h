@@ -157,7 +157,8 @@ int tpr_reduce_noalloc(const tpr_reduce_desc* desc, const void* in, void* out, v
  * only) are dense over the kept dims, as tpr_reduce writes them; `in` (x) is
  * read by VAR / STD only; grad_in is written dense row-major over sizes.  VAR
  * and STD recompute the mean with tpr_reduce into the workspace; MEAN divides
- * grad_out by the count there, once per output. */
+ * grad_out by the count once per output, there or in the kernel (rows of a
+ * reduced innermost dim). */
 size_t tpr_reduce_backward_workspace_bytes(const tpr_reduce_desc* desc);
 int tpr_reduce_backward(const tpr_reduce_desc* desc, const void* grad_out, const void* in, const void* result,
                         void* grad_in, void* workspace, size_t workspace_bytes, void* stream);
@@ -195,7 +196,7 @@ int tpr_topk_plan(int32_t dtype, int64_t rows, int64_t cols, int64_t k, int64_t 
 
 /* Top-k / top-p (nucleus) sampling of one token id per row of float32 logits
  * (a consumer of tpr_topk; TensorPlay has no sampler, so the definition is
- * this build's): for the k largest logits of a row, sorted v_0 >= ... >=
+ * this library's): for the k largest logits of a row, sorted v_0 >= ... >=
  * v_{k-1} (ties to the lowest index, as tpr_topk),
  *   p_j = exp(v_j / T - v_0 / T),  c_j = p_0 + ... + p_j,
  *   m   = the first j with c_j >= top_p * c_{k-1},
@@ -206,7 +207,8 @@ int tpr_topk_plan(int32_t dtype, int64_t rows, int64_t cols, int64_t k, int64_t 
  * tpr_sample_workspace_bytes: for k <= 1024 tpr_topk's (the draw runs in
  * top-k's last phase, nothing else is written); for k > 1024 tpr_topk's and
  * room for k sorted values and indices per row, which must be there but is not
- * written (the draw finds its position by weight, without sorting). */
+ * written (the draw finds its position by weight, without sorting).  Weights are
+ * float32 exponentials, their sums float64 or 64-bit fixed point for k > 1024. */
 size_t tpr_sample_workspace_bytes(int32_t dtype, int64_t rows, int64_t cols, int64_t k);
 int tpr_sample(const void* logits, int32_t dtype, int64_t rows, int64_t cols, int64_t row_stride, int64_t k,
                float temperature, float top_p, const float* uniforms, int64_t* out_ids, void* workspace,

@@ -9,8 +9,9 @@
 //  * sums accumulate in fp64 (the reference's full sum does, :30/:94; its dim
 //    sum accumulates in fp32, :168, which is less accurate -- the result here is
 //    closer to the exact sum than the reference's);
-//  * var/std use a Welford/Chan merge of per-thread shifted sums instead of the
-//    reference's five-pass mean/sub/mul/sum/div composite (:817-855).
+//  * var/std use one pass of shifted sums instead of the reference's five-pass
+//    mean/sub/mul/sum/div composite (:817-855): one shift per output up to 2^24
+//    elements (ShiftVarOp), per-thread shifts with a Welford/Chan merge above.
 //
 // Layout classes after the host canonicalises the view (drop size-1 dims, merge
 // adjacent dims that are contiguous with each other and share reduce status):
@@ -20,9 +21,10 @@
 //   runs    several reduced dims, or kept dims that do not merge, the innermost
 //           reduced dim contiguous            -> k_runs   (128-bit loads along the runs)
 //   general anything else                    -> k_general (index arithmetic)
-// Any of them may split the reduced extent over S workgroups; the S partial
-// states then go through k_finalize (no atomics; fixed combine order, so results
-// are deterministic run to run).
+// Any of them may split the reduced extent over S workgroups.  The S partial
+// states combine in a fixed order, so results are deterministic run to run: in the
+// same launch by the workgroup that draws the last ticket (split_finish; atomics
+// carry the states and count the tickets, no sum), or in k_finalize.
 
 #include <hip/hip_runtime.h>
 
@@ -1438,8 +1440,9 @@ int validate(const tpr_reduce_desc* d) {
 
 constexpr long long kFewCols = 128;  // most columns of k_few_cols
 
-// Splits of a few-columns plan: about four workgroups per CU, at least two rounds
-// of four vectors per thread (a split costs a finalize launch).
+// Splits of a few-columns plan: up to four workgroups per CU, with at least two
+// rounds of four vectors per thread each, as a split has states to publish and fold
+// (uint8 [64, 224, 224, 3]: S = 4, one workgroup per CU).
 void plan_few_cols(Plan& p, int NV) {
     const long long want = (long long)device_info().cus * 4;
     const long long T = kBlock / p.inner * p.inner;

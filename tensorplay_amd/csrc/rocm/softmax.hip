@@ -2258,9 +2258,12 @@ bool rows_path(const tpr_softmax_desc* d) {
            knobs().general == 0;
 }
 
-// Workspace of the split-row kernels (zero when they are not used): one float2
-// per (row, chunk).  Independent of pointer alignment: it assumes the scalar
-// single-pass capacity (16384 floats forward, 4096 backward).
+// Workspace of the split-row kernels: one float2 per (row, chunk).  Independent of
+// pointer alignment and stream, so more rows ask for it than use it: rows of up to
+// 32768 floats stay in registers (gradients ask from 4097 on, forward rows from
+// 16385), and longer ones take pieces where nothing is captured or aliased.  The
+// figure is part of the interface: programs keep buffers of it, and a call with
+// less is refused.
 size_t smx_workspace(const tpr_softmax_desc* d) {
     if (d->dtype == TPR_FLOAT64 || !rows_path(d) || d->outer == 0 || d->n == 0) return 0;
     const bool bw = d->mode >= TPR_SOFTMAX_BWD;

@@ -277,8 +277,9 @@ __device__ void sample_from_sel(const TopkArgs& a, long long row, const float* p
 
 // Workspace that tpr_sample asks for with k > kKMax: tpr_topk's own, then room
 // for sorted values [rows][k] (float32) and indices [rows][k] (int64), each
-// part on a 256-byte boundary.  The draw no longer sorts, but callers size
-// buffers they keep by this figure and a smaller one stays an error.
+// part on a 256-byte boundary.  The draw no longer sorts and writes none of it.
+// The figure is part of the interface all the same: the query keeps its answer, and
+// a call with less stays refused.
 inline size_t round_up_256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 inline size_t sample_sorted_bytes(int64_t rows, int64_t cols, int64_t k) {
